@@ -10,6 +10,7 @@
 
 #include "../../include/fgw_mha.h"
 #include "fmha_aux.h"
+#include "fmha_decode.h"
 #include "fmha_kernel.h"
 #include "fmha_prefill.h"
 #include "fmha_registry.h"
@@ -26,6 +27,9 @@ FGW_MHA_FOR_PREFILL_LO(FGW_MHA_EXTERN_PREFILL, true)
 FGW_MHA_FOR_PREFILL_HI(FGW_MHA_EXTERN_PREFILL, true)
 FGW_MHA_FOR_PREFILL_LO(FGW_MHA_EXTERN_PREFILL, false)
 FGW_MHA_FOR_PREFILL_HI(FGW_MHA_EXTERN_PREFILL, false)
+
+FGW_MHA_FOR_DECODE(FGW_MHA_EXTERN_DECODE, true)
+FGW_MHA_FOR_DECODE(FGW_MHA_EXTERN_DECODE, false)
 
 #define FGW_ENTRY(BF, DP, LY) \
   if (bf16 == BF && dpad == DP && layout == LY) return FwdEntry{&launch_fwd<BF, DP, LY>, &occupancy_fwd<BF, DP, LY>};
@@ -48,6 +52,14 @@ FwdEntry fwd_entry(bool bf16, int dpad, int layout, int stages) {
   FGW_MHA_FOR_PREFILL_LO(FGW_PREFILL_ENTRY, false)
   FGW_MHA_FOR_PREFILL_HI(FGW_PREFILL_ENTRY, false)
   return FwdEntry{nullptr, nullptr};
+}
+
+FwdLaunchFn decode_entry(bool bf16, int dpad) {
+#define FGW_DECODE_ENTRY(BF, DP) \
+  if (bf16 == BF && dpad == DP) return &launch_decode<BF, DP>;
+  FGW_MHA_FOR_DECODE(FGW_DECODE_ENTRY, true)
+  FGW_MHA_FOR_DECODE(FGW_DECODE_ENTRY, false)
+  return nullptr;
 }
 
 hipError_t launch_merge(bool bf16, const MergeParams& p, hipStream_t stream) {
@@ -477,7 +489,12 @@ int launch_partial_kernel(const fgw_mha_shape* s, const fgw_mha_plan_t* p,
   FwdParams f = make_params(s, p, t, mode);
   f.split_direct = whole && mode == 1 && tile_balanced(p->layout, s->causal, p->split_keys);
   f.arrivals = mode == 1 ? arrivals : nullptr;
-  const hipError_t err = e.launch(f, p->grid, stream);
+  const FwdLaunchFn launch = p->layout == kLayoutKey && s->sq == 1 &&
+                                         decode_takes(p->dim_padded, (int64_t)s->heads * s->dim * 2,
+                                                      s->page_size)
+                                 ? decode_entry(s->dtype == FGW_MHA_BFLOAT16, p->dim_padded)
+                                 : e.launch;
+  const hipError_t err = launch(f, p->grid, stream);
   return err == hipSuccess ? FGW_MHA_OK : hip_fail(err, "forward kernel launch");
 }
 

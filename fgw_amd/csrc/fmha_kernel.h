@@ -149,6 +149,43 @@ __device__ __forceinline__ int xcd_remap(int bid, int grid) {
   return xcd < r ? xcd * (q + 1) + local : r * (q + 1) + (xcd - r) * q + local;
 }
 
+// The work items of one program of the key layout: first, first + step, ...
+// The programs of one XCD (hardware: workgroup i runs on XCD i % 8) share one
+// contiguous range of the items, interleaved, so that at any time the XCD
+// reads neighbouring items. A balanced plan with fewer live items than
+// programs uses the first `work` programs, which lie on every XCD.
+struct ProgramItems {
+  int first, step, count;
+};
+__device__ __forceinline__ ProgramItems key_items(int work) {
+  const int active = work < (int)gridDim.x ? work : (int)gridDim.x;
+  if ((int)blockIdx.x >= active) return ProgramItems{0, 1, 0};
+  const int xcd = (int)blockIdx.x % kNumXcd, local = (int)blockIdx.x / kNumXcd;
+  const int q8 = active / kNumXcd, r8 = active % kNumXcd;
+  const int nx = q8 + (xcd < r8 ? 1 : 0);           // programs on this XCD
+  const int sx = xcd * q8 + (xcd < r8 ? xcd : r8);  // first of them in program order
+  const int per = work / active, rem = work % active;
+  const int a = sx * per + (sx < rem ? sx : rem);
+  const int end = (sx + nx) * per + (sx + nx < rem ? sx + nx : rem);
+  return ProgramItems{a + local, nx, local < end - a ? (end - a - local + nx - 1) / nx : 0};
+}
+
+// Whether a work item of the key layout loads K/V non-temporally: nothing
+// else of the call reads its rows again (one query tile, and head rows that
+// fill whole 128-byte lines, which heads would otherwise share), and a batch
+// of requests of its length is too large for the 256 MB last-level cache to
+// keep until the next call. Large reads then gain what the cache's
+// allocations cost; below that size repeated calls find their K/V there.
+// Measured over three rotating sets of inputs, the time non-temporal over
+// plain: B8 H8 D128 KV 512 / 1024 / 2048 (16 / 32 / 64 MiB) 1.20 / 1.29 /
+// 1.07, KV 3072 (96 MiB) 0.99, KV 4096-8192 (128-256 MiB) 0.89-0.90; D 16 and
+// 48 (shared lines) 1.45 and 1.11; two query tiles 1.21.
+constexpr int64_t kNonTemporalBytes = int64_t(128) << 20;
+__device__ __forceinline__ bool non_temporal_kv(const FwdParams& p, int len, int64_t row_bytes) {
+  return p.q_tiles == 1 && p.dim % 64 == 0 &&
+         2 * (int64_t)len * p.batch * row_bytes >= kNonTemporalBytes;
+}
+
 template <int A, int B>
 struct CMax {
   static constexpr int value = A > B ? A : B;
@@ -204,7 +241,6 @@ struct Cfg {
   static_assert(TILE_BYTES % 1024 == 0 && INSTR % NWQ == 0 && 64 % CPR == 0, "DMA granularity");
   static_assert(NBUF == 1 || NBUF == 2, "one or two K/V stages per key group");
   static_assert(LDS_BYTES <= kLdsBudget, "LDS budget of one CU");
-  static_assert(kMaxBalancedBatch % 64 == 0, "balanced-split prefix scan: whole lanes");
 };
 
 // LDS DMA (global_load_lds_dwordx4) for kernels that place their own waits
@@ -729,47 +765,48 @@ __device__ __forceinline__ int balanced_splits(int len, int split_keys, int spli
 }
 
 // Exclusive prefix sums of the balanced split counts over the batch, into
-// pre[0 .. B] (pre[B] = total), by the first wave of the workgroup: lane l
-// takes requests [16 l, 16 l + 16) (B <= 1024), the lane sums are scanned
-// across the wave with shuffles, then every lane writes its requests' prefix
-// sums. Every thread of the workgroup calls it (it ends with a barrier).
-template <class C>
-__device__ void balanced_prefix(const FwdParams& p, const int32_t* lengths, int capacity,
-                                int32_t* pre, int wave, int lane) {
+// pre[0 .. B] (pre[B] = total), by the first wave of the workgroup: 64 requests
+// at a time, one per lane, scanned across the wave with shuffles. Every
+// thread of the workgroup calls it (it ends with a barrier).
+__device__ __forceinline__ void balanced_prefix(const FwdParams& p, const int32_t* lengths,
+                                                int capacity, int32_t* pre, int wave, int lane) {
   if (wave == 0) {
-    constexpr int kPer = kMaxBalancedBatch / 64;
-    const int b0 = lane * kPer;
-    int cnt[kPer];
-    int local = 0;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int b = b0 + i;
+    int base = 0;
+    for (int b0 = 0; b0 < p.batch; b0 += 64) {
+      const int b = b0 + lane;
       int c = 0;
       if (b < p.batch) {
         int len = lengths[b];
         len = len < 0 ? 0 : (len > capacity ? capacity : len);
         c = balanced_splits(len, p.split_keys, p.splits);
       }
-      cnt[i] = c;
-      local += c;
-    }
-    int incl = local;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int up = __shfl_up(incl, off, 64);
-      incl += lane >= off ? up : 0;
-    }
-    int run = incl - local;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      if (b0 + i < p.batch) {
-        pre[b0 + i] = run;
-        run += cnt[i];
+      int incl = c;
+      for (int off = 1; off < 64; off <<= 1) {
+        const int up = __shfl_up(incl, off, 64);
+        incl += lane >= off ? up : 0;
       }
+      if (b < p.batch) pre[b] = base + incl - c;
+      base += __shfl(incl, 63, 64);
     }
-    if (lane == 63) pre[p.batch] = incl;
+    if (lane == 0) pre[p.batch] = base;
   }
   __syncthreads();
+}
+
+// The request of balanced work-item group g (pre[b] <= g < pre[b + 1]; pre is
+// strictly increasing: every request has at least one split), with g's split
+// and the request's split count.
+__device__ __forceinline__ int balanced_request(const int32_t* pre, int batch, int g, int& split,
+                                                int& nsplit) {
+  int lo = 0, hi = batch;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (__builtin_amdgcn_readfirstlane(pre[mid]) <= g) lo = mid; else hi = mid;
+  }
+  const int pb = __builtin_amdgcn_readfirstlane(pre[lo]);
+  split = g - pb;
+  nsplit = __builtin_amdgcn_readfirstlane(pre[lo + 1]) - pb;
+  return lo;
 }
 
 // LSE merge of the split partials of output rows [q0, q0 + rows) of (b, h),
@@ -1027,7 +1064,6 @@ constexpr int kFusedMergeMaxChunk = DPAD == 32 ? 8 : kMergeChunk;
 template <bool BF16, int THREADS, int ROWS_TILE, int MAXCH>
 __device__ void arrive_and_merge(const FwdParams& p, int b, int h, int qt, int used,
                                  unsigned char* lds, int tid) {
-  static_assert(THREADS == kMergeThreads, "the merge runs on one kMergeThreads workgroup");
   wait_vm<0>();     // this wave's partial rows and LSE are complete at the device
   __syncthreads();  // ... and every wave's
   int* flag = reinterpret_cast<int*>(lds);
@@ -1049,7 +1085,7 @@ __device__ void arrive_and_merge(const FwdParams& p, int b, int h, int qt, int u
   const int q0 = qt * ROWS_TILE;
   const int rows = sq - q0 < ROWS_TILE ? sq - q0 : ROWS_TILE;
   merge_rows<BF16, MAXCH, true>(p.parts, p.lse, p.out, sq, heads, dim, slots, used, b, h, q0,
-                                rows, tid, kMergeThreads);
+                                rows, tid, THREADS);
   if (tid == 0) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -1101,8 +1137,8 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
   int work = p.work;
   if constexpr (C::LAYOUT == kLayoutKey) {
     if (balanced) {
-      balanced_prefix<C>(p, lengths, capacity, reinterpret_cast<int32_t*>(smem + C::PREFIX_OFF),
-                         wave, lane);
+      balanced_prefix(p, lengths, capacity, reinterpret_cast<int32_t*>(smem + C::PREFIX_OFF), wave,
+                      lane);
       work = __builtin_amdgcn_readfirstlane(pre[p.batch]) * p.heads * p.q_tiles;
     }
   }
@@ -1140,19 +1176,10 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
       // Segments a host plan cannot produce are skipped whole (uniform).
       if (w < 0 || w >= tasks || slot >= p.slots || sg[1] < 0 || sg[2] < 0) continue;
     } else if (balanced) {
-      // g = w / (H q_tiles) = pre[b] + split for the request b with
-      // pre[b] <= g < pre[b + 1] (pre is strictly increasing: every request
-      // has at least one split); the rest of w is (h, q tile).
+      // g = w / (H q_tiles) = pre[b] + split; the rest of w is (h, q tile).
       const int hq = p.heads * p.q_tiles;
       const int g = w / hq;
-      int lo = 0, hi = p.batch;
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (__builtin_amdgcn_readfirstlane(pre[mid]) <= g) lo = mid; else hi = mid;
-      }
-      const int pb = __builtin_amdgcn_readfirstlane(pre[lo]);
-      split = g - pb;
-      nsplit = __builtin_amdgcn_readfirstlane(pre[lo + 1]) - pb;
+      const int lo = balanced_request(pre, p.batch, g, split, nsplit);
       w = lo * hq + w % hq;
     } else {
       split = w % p.splits;

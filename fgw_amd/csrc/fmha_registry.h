@@ -25,6 +25,8 @@ inline int dim_tile(int dim) {
 // The kernel of (dtype, head-dim tile, layout, stages); stages 0 is the
 // instantiation's default, 1 the key layout's single-stage variant (tile 128).
 FwdEntry fwd_entry(bool bf16, int dpad, int layout, int stages = 0);
+// The key layout's kernel of (dtype, head-dim tile) for Sq = 1.
+FwdLaunchFn decode_entry(bool bf16, int dpad);
 hipError_t launch_merge(bool bf16, const MergeParams& p, hipStream_t stream);
 hipError_t launch_gather(const GatherParams& p, hipStream_t stream);
 hipError_t launch_pack(const PackParams& p, int total_pages, hipStream_t stream);
@@ -56,6 +58,12 @@ hipError_t launch_group_merge(bool bf16, const GroupMergeParams& p, int groups, 
 #define FGW_MHA_EXTERN_PREFILL(BF, DP)                                               \
   extern template hipError_t launch_prefill<BF, DP>(const FwdParams&, int, hipStream_t); \
   extern template int occupancy_prefill<BF, DP>();
+// The key layout's single-token kernel (Sq = 1), every head-dim tile.
+#define FGW_MHA_FOR_DECODE(X, BF) X(BF, 32) X(BF, 64) X(BF, 128) X(BF, 256)
+#define FGW_MHA_INSTANTIATE_DECODE(BF, DP) \
+  template hipError_t launch_decode<BF, DP>(const FwdParams&, int, hipStream_t);
+#define FGW_MHA_EXTERN_DECODE(BF, DP) \
+  extern template hipError_t launch_decode<BF, DP>(const FwdParams&, int, hipStream_t);
 #define FGW_MHA_EXTERN(BF, DP)                                                                     \
   extern template hipError_t launch_fwd<BF, DP, kLayoutQuery>(const FwdParams&, int, hipStream_t); \
   extern template hipError_t launch_fwd<BF, DP, kLayoutKey>(const FwdParams&, int, hipStream_t);   \
