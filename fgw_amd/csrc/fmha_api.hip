@@ -28,6 +28,8 @@ FGW_MHA_FOR_PREFILL_HI(FGW_MHA_EXTERN_PREFILL, true)
 FGW_MHA_FOR_PREFILL_LO(FGW_MHA_EXTERN_PREFILL, false)
 FGW_MHA_FOR_PREFILL_HI(FGW_MHA_EXTERN_PREFILL, false)
 
+FGW_MHA_FOR_PREFILL_ROWS(FGW_MHA_EXTERN_PREFILL_ROWS, true)
+FGW_MHA_FOR_PREFILL_ROWS(FGW_MHA_EXTERN_PREFILL_ROWS, false)
 FGW_MHA_FOR_DECODE(FGW_MHA_EXTERN_DECODE, true)
 FGW_MHA_FOR_DECODE(FGW_MHA_EXTERN_DECODE, false)
 
@@ -52,6 +54,14 @@ FwdEntry fwd_entry(bool bf16, int dpad, int layout, int stages) {
   FGW_MHA_FOR_PREFILL_LO(FGW_PREFILL_ENTRY, false)
   FGW_MHA_FOR_PREFILL_HI(FGW_PREFILL_ENTRY, false)
   return FwdEntry{nullptr, nullptr};
+}
+
+FwdLaunchFn prefill_rows_entry(bool bf16, int dpad, int rows) {
+#define FGW_PREFILL_ROWS_ENTRY(BF, DP, RM) \
+  if (bf16 == BF && dpad == DP && rows == RM) return &launch_prefill<BF, DP, RM>;
+  FGW_MHA_FOR_PREFILL_ROWS(FGW_PREFILL_ROWS_ENTRY, true)
+  FGW_MHA_FOR_PREFILL_ROWS(FGW_PREFILL_ROWS_ENTRY, false)
+  return nullptr;
 }
 
 FwdLaunchFn decode_entry(bool bf16, int dpad) {
@@ -478,6 +488,23 @@ int check_schedule(const fgw_mha_shape* s, const fgw_mha_schedule* sc) {
   return FGW_MHA_OK;
 }
 
+// The kernel of a plan: the layout's own (`fallback`) or one of its variants.
+// - Key layout, Sq = 1: the single-token kernel where decode_takes it.
+// - Prefill layout: a row-group variant where the whole-block fast path would
+//   not hold (pages that a 64-key block straddles, or a head dim below its
+//   tile) and an instruction's rows (512 / tile of them) still lie in one page.
+FwdLaunchFn kernel_of(const fgw_mha_shape* s, const fgw_mha_plan_t* p, FwdLaunchFn fallback) {
+  const bool bf16 = s->dtype == FGW_MHA_BFLOAT16;
+  FwdLaunchFn f = nullptr;
+  if (p->layout == kLayoutKey && s->sq == 1 &&
+      decode_takes(p->dim_padded, (int64_t)s->heads * s->dim * 2, s->page_size))
+    f = decode_entry(bf16, p->dim_padded);
+  else if (p->layout == kLayoutPrefill && (s->page_size % 64 || s->dim != p->dim_padded) &&
+           s->page_size % (512 / p->dim_padded) == 0)
+    f = prefill_rows_entry(bf16, p->dim_padded, s->dim == p->dim_padded ? kRowsGroup : kRowsPadded);
+  return f ? f : fallback;
+}
+
 // `whole`: the partial kernel of a full call, whose merge follows (a
 // tile-balanced plan's one-split tiles then write their output directly).
 int launch_partial_kernel(const fgw_mha_shape* s, const fgw_mha_plan_t* p,
@@ -489,11 +516,7 @@ int launch_partial_kernel(const fgw_mha_shape* s, const fgw_mha_plan_t* p,
   FwdParams f = make_params(s, p, t, mode);
   f.split_direct = whole && mode == 1 && tile_balanced(p->layout, s->causal, p->split_keys);
   f.arrivals = mode == 1 ? arrivals : nullptr;
-  const FwdLaunchFn launch = p->layout == kLayoutKey && s->sq == 1 &&
-                                         decode_takes(p->dim_padded, (int64_t)s->heads * s->dim * 2,
-                                                      s->page_size)
-                                 ? decode_entry(s->dtype == FGW_MHA_BFLOAT16, p->dim_padded)
-                                 : e.launch;
+  const FwdLaunchFn launch = kernel_of(s, p, e.launch);
   const hipError_t err = launch(f, p->grid, stream);
   return err == hipSuccess ? FGW_MHA_OK : hip_fail(err, "forward kernel launch");
 }

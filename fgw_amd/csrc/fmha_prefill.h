@@ -81,10 +81,16 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-template <bool BF16_, int DPAD_>
+// ROWS: how the DMA finds a block's rows. kRowsBlock: blocks that lie in one
+// page, at D == DPAD; others take the per-key path. kRowsGroup: the page table
+// is resolved per DMA instruction, for pages that blocks may straddle.
+// kRowsPadded: likewise, for D < DPAD.
+enum RowsMode : int { kRowsBlock = 0, kRowsGroup = 1, kRowsPadded = 2 };
+template <bool BF16_, int DPAD_, int ROWS_ = kRowsBlock>
 struct PCfg {
   static constexpr bool BF16 = BF16_;
   static constexpr int DPAD = DPAD_;
+  static constexpr int ROWS = ROWS_;
   static constexpr int LAYOUT = kLayoutPrefill;
   static constexpr int NWQ = 8;  // waves along query rows; all share each K/V block
   static constexpr int NWK = 1;
@@ -112,6 +118,7 @@ struct PCfg {
   static constexpr int KSW = CMin<16, CPR>::value;
   static constexpr int VSW = CPR / 4;
   static constexpr int RPI = 64 / CPR;
+  static constexpr int WINDOW = ROWS != kRowsBlock ? 64 / INSTR_PER_WAVE : 64;  // blocks per offset window
   static_assert(DPAD == 64 || DPAD == 128, "prefill layout head-dim tiles");
   static_assert(NKSLOT == 4 && NVSLOT == 4, "matrix phases take slots n % 4");
   static_assert(INSTR % NWQ == 0 && INSTR_PER_WAVE >= 1, "DMA granularity");
@@ -154,8 +161,39 @@ __device__ __forceinline__ int64_t block_offset(const FwdParams& p, const int32_
   return block_offset_of<C>(p, block_page_id<C>(p, table_b, key0, j), row_bytes, key0, N, len, j);
 }
 
-// Offsets of blocks [64 w, 64 w + 64) of a work item, one per lane (lane l:
-// block 64 w + l).
+// Pool byte offset of the rows of DMA instruction q of this wave in block
+// j (rows [RPI i, RPI i + RPI), i = q NWQ + wave; page_size % RPI == 0, so they
+// lie in one page), or -1 when they need the per-key path (they straddle len
+// or leave the pool). Evaluated per lane.
+template <class C>
+__device__ __forceinline__ int64_t row_group_offset(const FwdParams& p, const int32_t* table_b,
+                                                    int64_t row_bytes, int key0, int N, int len,
+                                                    int j, int q, int wave) {
+  const u32 pos0 = (u32)key0 + (u32)j * C::BN + (u32)(C::RPI * (q * C::NWQ + wave));
+  const u32 pg = div_page(pos0, p.page_magic, p.page_shift);
+  const u32 last = (u32)p.width - 1u;
+  const int32_t id = table_b[pg < last ? pg : last];
+  const int64_t row0 = (int64_t)id * p.page_size + (pos0 - pg * (u32)p.page_size);
+  const bool fast = j < N && (int64_t)pos0 + C::RPI <= len && row0 >= 0 &&
+                    row0 + C::RPI <= p.pool_rows;
+  return fast ? row0 * row_bytes : -1;
+}
+
+// Window w of per-lane offsets: block WINDOW w + lane, or (row groups) instruction
+// lane % INSTR_PER_WAVE of block WINDOW w + lane / INSTR_PER_WAVE.
+template <class C>
+__device__ __forceinline__ int64_t window_offset(const FwdParams& p, const int32_t* table_b,
+                                                 int64_t row_bytes, int key0, int N, int len,
+                                                 int w, int wave, int lane) {
+  if constexpr (C::ROWS != kRowsBlock)
+    return row_group_offset<C>(p, table_b, row_bytes, key0, N, len,
+                               C::WINDOW * w + lane / C::INSTR_PER_WAVE, lane % C::INSTR_PER_WAVE,
+                               wave);
+  else
+    return block_offset<C>(p, table_b, row_bytes, key0, N, len, C::WINDOW * w + lane);
+}
+
+// Window w of a work item's offsets, one per lane (window_offset).
 struct BlockWindow {
   int w;
   int64_t off;
@@ -171,17 +209,19 @@ __device__ __forceinline__ int64_t readlane64(int64_t x, int lane) {
 // when the block is not in the fast case: every key row is resolved through
 // the table and masked chunks (key >= len, d >= D, page id outside the
 // pool) read the zero chunk. Instruction q of the wave fills LDS
-// [dst + 1024 i, + 1024) with i = q * NWQ + wave.
+// [dst + 1024 i, + 1024) with i = q * NWQ + wave; only_q >= 0: instruction only_q alone.
 template <class C, bool IS_V>
 __device__ __forceinline__ void issue_slow_tile(const FwdParams& p, const int32_t* table_b,
                                                 const char* base, int64_t row_bytes, int pos0,
-                                                int len, u32 dst, int wave, int lane) {
+                                                int len, u32 dst, int wave, int lane,
+                                                int only_q = -1) {
   const u32 page = (u32)p.page_size;
   const int dim = opaque_uniform(p.dim);
   lane = opaque_lane(lane);
   const char* zero = reinterpret_cast<const char*>(kZeroChunk);
 #pragma unroll
   for (int q = 0; q < C::INSTR_PER_WAVE; ++q) {
+    if (only_q >= 0 && q != only_q) continue;
     const int i = q * C::NWQ + wave;
     const int r = C::RPI * i + lane / C::CPR, pos_in_row = lane % C::CPR;
     const int pos = pos0 + r;
@@ -223,6 +263,36 @@ __device__ __forceinline__ void issue_fast_block(const char* kbase, const char* 
   for (int q = 0; q < C::INSTR_PER_WAVE; ++q) {
     dma_saddr(kbase, bd.k[q], kw + 1024u * (u32)(q * C::NWQ));
     dma_saddr(vbase, bd.v[q], vw + 1024u * (u32)(q * C::NWQ));
+  }
+}
+
+// kRowsGroup / kRowsPadded: the per-lane byte offsets of the wave's DMA
+// instructions from their own first row, and (kRowsPadded) whether the lane's
+// chunk lies below D; the other lanes read the zero chunk.
+template <class C>
+struct RowDma {
+  u32 k[C::INSTR_PER_WAVE], v[C::INSTR_PER_WAVE];
+  bool k_live[C::INSTR_PER_WAVE], v_live[C::INSTR_PER_WAVE];
+  __device__ __forceinline__ RowDma(const DmaLanes<C>& dl, int dim, int wave, int lane) {
+#pragma unroll
+    for (int q = 0; q < C::INSTR_PER_WAVE; ++q) {
+      k[q] = dl.kq(q, wave);
+      v[q] = dl.vq(q, wave);
+      const int r = C::RPI * (q * C::NWQ + wave) + lane / C::CPR, pos = lane % C::CPR;
+      k_live[q] = C::ROWS != kRowsPadded || (pos ^ (r % C::KSW)) * 8 < dim;
+      v_live[q] = C::ROWS != kRowsPadded || (pos ^ (4 * (r % C::VSW))) * 8 < dim;
+    }
+  }
+};
+
+// One DMA instruction of rows that start at the uniform address `base`.
+template <class C>
+__device__ __forceinline__ void issue_row_group(const char* base, u32 voff, bool live, u32 dst) {
+  if constexpr (C::ROWS == kRowsPadded) {
+    const char* zero = reinterpret_cast<const char*>(kZeroChunk);
+    dma_flat(live ? base + voff : zero, dst);
+  } else {
+    dma_saddr(base, voff, dst);
   }
 }
 
@@ -363,6 +433,7 @@ __global__ __launch_bounds__(C::THREADS) void prefill_kernel(FwdParams p_arg,
   const int64_t row_bytes = (int64_t)p.heads * p.dim * 2;
   const DmaLanes<C> dl(lane, wave, row_bytes);
   const BlockDma<C> bd(dl, wave, row_bytes);
+  const RowDma<C> rd(dl, p.dim, wave, lane);
 
   // Work items: the programs of one XCD (hardware: workgroup i runs on XCD
   // i % 8) share one contiguous range of the items, interleaved: program
@@ -588,7 +659,9 @@ __global__ __launch_bounds__(C::THREADS) void prefill_kernel(FwdParams p_arg,
       // guess held) waits only for that load and not for Q behind it.
       const OperandAddr<C> ad_q(ln, kring_lds, vring_lds);
       BlockWindow win0{0, 0};
-      if (key0 == key0_full)
+      if constexpr (C::ROWS != kRowsBlock)
+        win0.off = window_offset<C>(p, table_b, row_bytes, key0, N, len, 0, wave, lane);
+      else if (key0 == key0_full)
         win0.off = block_offset_of<C>(p, id_first, row_bytes, key0, N, len, lane);
       else
         win0.off = block_offset<C>(p, table_b, row_bytes, key0, N, len, lane);
@@ -596,14 +669,31 @@ __global__ __launch_bounds__(C::THREADS) void prefill_kernel(FwdParams p_arg,
       // K and V of block j < N into K slot j % 4, V slot j % 4 (jslot: an
       // int, or a compile-time constant in the unrolled loops).
       auto issue_block = [&](int j, auto jslot) {
-        if ((j >> 6) != win0.w) {  // uniform: the block entered the next window
+        if (j / C::WINDOW != win0.w) {  // uniform: the block entered the next window
           win0 = win1;
-          win1 = BlockWindow{win0.w + 1, block_offset<C>(p, table_b, row_bytes, key0, N, len,
-                                                         64 * (win0.w + 1) + lane)};
+          win1 = BlockWindow{win0.w + 1, window_offset<C>(p, table_b, row_bytes, key0, N, len,
+                                                          win0.w + 1, wave, lane)};
         }
-        const int64_t off = readlane64(win0.off, j & 63);
         const u32 kdst = kring_lds + (u32)((int)jslot * C::TILE_BYTES);
         const u32 vdst = vring_lds + (u32)((int)jslot * C::TILE_BYTES);
+        if constexpr (C::ROWS != kRowsBlock) {
+#pragma unroll
+          for (int q = 0; q < C::INSTR_PER_WAVE; ++q) {
+            const int64_t off = readlane64(win0.off, j % C::WINDOW * C::INSTR_PER_WAVE + q);
+            const u32 at = 1024u * (u32)(q * C::NWQ + wave);
+            if ((int32_t)((uint64_t)off >> 32) >= 0) {
+              issue_row_group<C>(kb + off, rd.k[q], rd.k_live[q], kdst + at);
+              issue_row_group<C>(vb + off, rd.v[q], rd.v_live[q], vdst + at);
+            } else {
+              int pos0 = key0 + j * C::BN;
+              asm volatile("" : "+s"(pos0));
+              issue_slow_tile<C, false>(p, table_b, kb, row_bytes, pos0, len, kdst, wave, lane, q);
+              issue_slow_tile<C, true>(p, table_b, vb, row_bytes, pos0, len, vdst, wave, lane, q);
+            }
+          }
+          return;
+        }
+        const int64_t off = readlane64(win0.off, j % C::WINDOW);
         if ((int32_t)((uint64_t)off >> 32) >= 0) {  // off >= 0 as a scalar compare
           issue_fast_block<C>(kb + off, vb + off, kdst, vdst, bd, wave);
         } else {
@@ -696,7 +786,7 @@ __global__ __launch_bounds__(C::THREADS) void prefill_kernel(FwdParams p_arg,
           qf[kk] = *(const __attribute__((address_space(3))) u32x4*)(lds_at(ad_q.k[kk]) + off);
       }
 
-      win1.off = block_offset<C>(p, table_b, row_bytes, key0, N, len, 64 + lane);
+      win1.off = window_offset<C>(p, table_b, row_bytes, key0, N, len, 1, wave, lane);
       // The wait for block 1, with the deferred stores (issued after block
       // 0's wait) in flight behind it.
       auto wait_block1 = [&]() {
@@ -824,9 +914,9 @@ __global__ __launch_bounds__(C::THREADS) void prefill_kernel(FwdParams p_arg,
   }
 }
 
-template <bool BF16, int DPAD>
+template <bool BF16, int DPAD, int ROWS = kRowsBlock>
 hipError_t launch_prefill(const FwdParams& p, int grid, hipStream_t stream) {
-  using C = PCfg<BF16, DPAD>;
+  using C = PCfg<BF16, DPAD, ROWS>;
   prefill_kernel<C><<<dim3(grid), dim3(C::THREADS), 0, stream>>>(p, p.table, p.lengths);
   return hipGetLastError();
 }

@@ -25,6 +25,8 @@ inline int dim_tile(int dim) {
 // The kernel of (dtype, head-dim tile, layout, stages); stages 0 is the
 // instantiation's default, 1 the key layout's single-stage variant (tile 128).
 FwdEntry fwd_entry(bool bf16, int dpad, int layout, int stages = 0);
+// The prefill layout's row-group kernel of (dtype, head-dim tile, rows mode).
+FwdLaunchFn prefill_rows_entry(bool bf16, int dpad, int rows);
 // The key layout's kernel of (dtype, head-dim tile) for Sq = 1.
 FwdLaunchFn decode_entry(bool bf16, int dpad);
 hipError_t launch_merge(bool bf16, const MergeParams& p, hipStream_t stream);
@@ -58,6 +60,13 @@ hipError_t launch_group_merge(bool bf16, const GroupMergeParams& p, int groups, 
 #define FGW_MHA_EXTERN_PREFILL(BF, DP)                                               \
   extern template hipError_t launch_prefill<BF, DP>(const FwdParams&, int, hipStream_t); \
   extern template int occupancy_prefill<BF, DP>();
+// The prefill layout's row-group variants (RowsMode in fmha_prefill.h): 1 for
+// pages that key blocks straddle, 2 for head dims below their tile.
+#define FGW_MHA_FOR_PREFILL_ROWS(X, BF) X(BF, 64, 1) X(BF, 128, 1) X(BF, 64, 2) X(BF, 128, 2)
+#define FGW_MHA_INSTANTIATE_PREFILL_ROWS(BF, DP, RM) \
+  template hipError_t launch_prefill<BF, DP, RM>(const FwdParams&, int, hipStream_t);
+#define FGW_MHA_EXTERN_PREFILL_ROWS(BF, DP, RM) \
+  extern template hipError_t launch_prefill<BF, DP, RM>(const FwdParams&, int, hipStream_t);
 // The key layout's single-token kernel (Sq = 1), every head-dim tile.
 #define FGW_MHA_FOR_DECODE(X, BF) X(BF, 32) X(BF, 64) X(BF, 128) X(BF, 256)
 #define FGW_MHA_INSTANTIATE_DECODE(BF, DP) \

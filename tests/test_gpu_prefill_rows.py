@@ -1,0 +1,74 @@
+"""The prefill layout's per-instruction variants against the oracle: pages that a
+64-key block straddles and head dims 80 and 96.
+
+Where they can go wrong: caches that end inside an instruction's rows, page
+sizes of one instruction's rows and off the powers of two, page ids outside
+the pool, more blocks than one window of offsets holds (32 at head-dim tile
+128, 64 at 64), several items per program (their output rows are deferred),
+fp32 partials of a head dim below its tile, causal rows without a key. Rows
+that no request reads hold NaN. The tolerance is the operator's (oracle
+TOLERANCES: the input type's rounding of P and O).
+"""
+import pytest
+import torch
+
+from oracle import mha_oracle as O
+
+gpu = pytest.mark.gpu
+
+
+def _check(b, sq, h, d, page, lengths, dtype, causal, outside=False, **plan):
+    from fgw_amd.operators.mha.current import build_kernel
+    width = -(-max(lengths) // page)
+    q, k, v, table = O.make_inputs(("rows", b, sq, h, d, page, width), 5, dtype)
+    lengths = torch.tensor(lengths, dtype=torch.int32)
+    k, v = O.poison_unread(k, v, table, lengths, page)
+    etable, ek, ev = table, k, v
+    if outside:  # the oracle reads a page of zeros where the kernel's id is invalid
+        table = table.clone()
+        table[0, 1], table[-1, 0] = -1, k.shape[0] // page
+        zeros = torch.zeros(page, h, d, dtype=dtype)
+        ek, ev = torch.cat([k, zeros]), torch.cat([v, zeros])
+        etable = table.clone()
+        etable[0, 1] = etable[-1, 0] = k.shape[0] // page
+    kern = build_kernel(b, sq, h, d, k.shape[0], width, page, causal,
+                        "float16" if dtype == torch.float16 else "bfloat16", 0, layout="prefill",
+                        **plan)
+    got = kern(*[x.cuda() for x in (q, k, v, table, lengths)]).cpu()
+    rtol, atol = O.TOLERANCES[dtype]
+    torch.testing.assert_close(got, O.chunked_reference(q, ek, ev, etable, lengths, page, causal),
+                               rtol=rtol, atol=atol)
+
+
+@gpu
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d,page,dtype", [
+    (128, 4, torch.bfloat16), (128, 16, torch.float16), (128, 48, torch.bfloat16),
+    (64, 8, torch.float16), (64, 32, torch.bfloat16), (96, 16, torch.bfloat16),
+    (96, 64, torch.float16), (80, 12, torch.float16), (80, 128, torch.bfloat16),
+    (128, 6, torch.bfloat16), (96, 5, torch.float16), (112, 16, torch.bfloat16)])
+def test_ragged_pages_match_the_oracle(d, page, dtype, causal):
+    lengths = [0, 1, 3, 63, 64, 65, 130, 257, 300]
+    for splits in (1, 2):
+        _check(len(lengths), 257, 2, d, page, lengths, dtype, causal, num_splits=splits)
+
+
+@gpu
+@pytest.mark.parametrize("d,page", [(128, 16), (64, 16), (96, 32)])
+def test_more_blocks_than_a_window(d, page):
+    _check(1, 300, 1, d, page, [4500], torch.bfloat16, False, num_splits=1)
+    _check(2, 260, 1, d, page, [4500, 2111], torch.bfloat16, True, num_splits=2)
+
+
+@gpu
+@pytest.mark.parametrize("d,page", [(96, 64), (128, 16), (80, 16)])
+def test_several_items_per_program(d, page):
+    for grid in (3, 8):
+        _check(2, 600, 3, d, page, [200, 333], torch.float16, False, num_splits=1,
+               persistent_programs=grid)
+
+
+@gpu
+@pytest.mark.parametrize("d,page", [(128, 16), (96, 64)])
+def test_page_ids_outside_the_pool_read_as_zeros(d, page):
+    _check(2, 200, 2, d, page, [320, 177], torch.bfloat16, False, outside=True, num_splits=1)
