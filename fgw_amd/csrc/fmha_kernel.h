@@ -82,6 +82,7 @@ constexpr float kLn2 = 0.6931471805599453f;
 constexpr float kNegBig = -1.0e30f;  // running-max floor and empty-split LSE
 constexpr float kSoftmaxSumBound = 8192.0f;  // lane row-sum bound before O/l are rescaled
 constexpr int kNumXcd = 8;
+constexpr int kNumCus = 256;
 constexpr int kLdsBudget = 160 * 1024;
 // Largest batch of a length-balanced split plan (FwdParams::split_keys > 0):
 // the per-request split prefix sums live in LDS.

@@ -72,3 +72,26 @@ def test_several_items_per_program(d, page):
 @pytest.mark.parametrize("d,page", [(128, 16), (96, 64)])
 def test_page_ids_outside_the_pool_read_as_zeros(d, page):
     _check(2, 200, 2, d, page, [320, 177], torch.bfloat16, False, outside=True, num_splits=1)
+
+
+@gpu
+@pytest.mark.parametrize("sq,lengths,plan", [
+    (2049, [2100, 2049], dict(num_splits=1)),                  # 9 tiles x 34 (b, h) > 256 items
+    (1030, [1030, 700], dict(num_splits=2)),                   # split items, Sq > len rows
+    (2049, [2100, 2049], dict(num_splits=4, split_keys=640)),  # tiles of 1 to 4 splits
+    (2049, [2100, 2049], dict(num_splits=1, persistent_programs=40)),
+])
+def test_more_causal_items_than_cus(sq, lengths, plan):
+    """Longest-first order: every item is done once, whatever the plan and grid."""
+    from fgw_amd.operators.mha.current import build_kernel
+    b, h, d, page = 2, 17, 64, 64
+    width = -(-max(lengths) // page)
+    q, k, v, table = O.make_inputs(("order", b, sq, h, d, page, width), 3, torch.float16)
+    lengths = torch.tensor(lengths, dtype=torch.int32)
+    kern = build_kernel(b, sq, h, d, k.shape[0], width, page, True, "float16", 0, layout="prefill",
+                        **plan)
+    assert kern.compute_work > 256
+    got = kern(*[x.cuda() for x in (q, k, v, table, lengths)]).cpu()
+    rtol, atol = O.TOLERANCES[torch.float16]
+    torch.testing.assert_close(got, O.chunked_reference(q, k, v, table, lengths, page, True),
+                               rtol=rtol, atol=atol)
