@@ -11,6 +11,7 @@
 #include "../../include/fgw_mha.h"
 #include "fmha_aux.h"
 #include "fmha_decode.h"
+#include "fmha_half.h"
 #include "fmha_kernel.h"
 #include "fmha_prefill.h"
 #include "fmha_registry.h"
@@ -30,6 +31,8 @@ FGW_MHA_FOR_PREFILL_HI(FGW_MHA_EXTERN_PREFILL, false)
 
 FGW_MHA_FOR_PREFILL_ROWS(FGW_MHA_EXTERN_PREFILL_ROWS, true)
 FGW_MHA_FOR_PREFILL_ROWS(FGW_MHA_EXTERN_PREFILL_ROWS, false)
+FGW_MHA_FOR_PREFILL_ROWS(FGW_MHA_EXTERN_HALF, true)
+FGW_MHA_FOR_PREFILL_ROWS(FGW_MHA_EXTERN_HALF, false)
 FGW_MHA_FOR_DECODE(FGW_MHA_EXTERN_DECODE, true)
 FGW_MHA_FOR_DECODE(FGW_MHA_EXTERN_DECODE, false)
 
@@ -61,6 +64,14 @@ FwdLaunchFn prefill_rows_entry(bool bf16, int dpad, int rows) {
   if (bf16 == BF && dpad == DP && rows == RM) return &launch_prefill<BF, DP, RM>;
   FGW_MHA_FOR_PREFILL_ROWS(FGW_PREFILL_ROWS_ENTRY, true)
   FGW_MHA_FOR_PREFILL_ROWS(FGW_PREFILL_ROWS_ENTRY, false)
+  return nullptr;
+}
+
+FwdLaunchFn half_entry(bool bf16, int dpad, int rows) {
+#define FGW_HALF_ENTRY(BF, DP, RM) \
+  if (bf16 == BF && dpad == DP && rows == RM) return &launch_half<BF, DP, RM>;
+  FGW_MHA_FOR_PREFILL_ROWS(FGW_HALF_ENTRY, true)
+  FGW_MHA_FOR_PREFILL_ROWS(FGW_HALF_ENTRY, false)
   return nullptr;
 }
 
@@ -505,6 +516,53 @@ FwdLaunchFn kernel_of(const fgw_mha_shape* s, const fgw_mha_plan_t* p, FwdLaunch
   return f ? f : fallback;
 }
 
+constexpr int kRowsHalfTile = HCfg<true, 128, kRowsGroup>::ROWS_TILE;
+
+// Key blocks on the critical path of a direct plan with query tiles of `rows`
+// rows whose items take `per_step` blocks at a time, at full table capacity:
+// the longest item or an even share of all of them (longest first), plus an
+// item's fixed cost (about five blocks) for each round.
+double critical_steps(const fgw_mha_shape* s, int rows, int per_step, double step_cost) {
+  const int64_t capacity = (int64_t)s->width * s->page_size;
+  const int q_tiles = (s->sq + rows - 1) / rows;
+  const int64_t tiles = (int64_t)s->batch * s->heads * q_tiles;
+  const int64_t rounds = (tiles + kNumCus - 1) / kNumCus;
+  auto steps = [&](int64_t vis) {
+    vis = vis < 0 ? 0 : (vis > capacity ? capacity : vis);
+    return (vis + 64 * per_step - 1) / (64 * per_step);
+  };
+  const int64_t longest = steps(capacity);
+  double path = (double)(rounds * longest);
+  if (s->causal) {
+    int64_t sum = 0;
+    for (int t = 0; t < q_tiles; ++t)
+      sum += steps(capacity - s->sq + ((int64_t)(t + 1) * rows < s->sq ? (t + 1) * rows : s->sq));
+    const double share = (double)sum * s->batch * s->heads / kNumCus;
+    path = share > (double)longest ? share : (double)longest;
+  }
+  return path * step_cost + 5.0 * (double)rounds;
+}
+
+// Whether a direct prefill-layout plan runs on the half-tile kernel (128 rows
+// per item, two key blocks per step): where its critical path is at least 5%
+// shorter. A step costs 1.3 blocks at head-dim tile 64 and 1.66 at 128 (twice
+// the K/V reads per row, and with the CUs evenly loaded a lower clock). The
+// times it comes from, 256-row items against half tiles (BF16, three rotating
+// sets of inputs): causal S4096 H16 D64 70.8 / 57.8 us, S8192 H8 D64 132 / 99,
+// S3000 H12 D64 53 / 37, S4096 H16 D128 94.5 / 89.9, B8 H8 Q257 KV 1152 D96
+// 33.8 / 28.7 (D128 31.6 / 28.9), B2 H4 Q4096 KV 2048 D128 46.0 / 44.7; left
+// alone: causal S2048 H32 D128 53.5 / 57.2, S4096 H32 D64 88 / 109, full
+// B2 H8 Q4096 KV 2048 D128 66 / 87. Above 512 tiles the 256-row items balance
+// by themselves.
+bool half_tiles(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
+  if (p->layout != kLayoutPrefill || p->num_splits > 1 ||
+      s->page_size % (512 / p->dim_padded) || p->query_tile_tasks > 2 * kNumCus)
+    return false;
+  const double step_cost = p->dim_padded == 64 ? 1.3 : 1.66;
+  return critical_steps(s, kRowsHalfTile, 2, step_cost) <
+         0.95 * critical_steps(s, 2 * kRowsHalfTile, 1, 1.0);
+}
+
 // `whole`: the partial kernel of a full call, whose merge follows (a
 // tile-balanced plan's one-split tiles then write their output directly).
 int launch_partial_kernel(const fgw_mha_shape* s, const fgw_mha_plan_t* p,
@@ -517,6 +575,17 @@ int launch_partial_kernel(const fgw_mha_shape* s, const fgw_mha_plan_t* p,
   f.split_direct = whole && mode == 1 && tile_balanced(p->layout, s->causal, p->split_keys);
   f.arrivals = mode == 1 ? arrivals : nullptr;
   const FwdLaunchFn launch = kernel_of(s, p, e.launch);
+  if (half_tiles(s, p)) {
+    // Twice the items; a plan with fewer programs than items keeps its grid.
+    f.q_tiles = (s->sq + kRowsHalfTile - 1) / kRowsHalfTile;
+    f.work = s->batch * s->heads * f.q_tiles;
+    const int grid = p->grid == p->work_items ? f.work : (p->grid < f.work ? p->grid : f.work);
+    const FwdLaunchFn half =
+        half_entry(s->dtype == FGW_MHA_BFLOAT16, p->dim_padded,
+                   s->dim == p->dim_padded ? kRowsGroup : kRowsPadded);
+    const hipError_t err = half(f, grid, stream);
+    return err == hipSuccess ? FGW_MHA_OK : hip_fail(err, "forward kernel launch");
+  }
   const hipError_t err = launch(f, p->grid, stream);
   return err == hipSuccess ? FGW_MHA_OK : hip_fail(err, "forward kernel launch");
 }

@@ -27,6 +27,8 @@ inline int dim_tile(int dim) {
 FwdEntry fwd_entry(bool bf16, int dpad, int layout, int stages = 0);
 // The prefill layout's row-group kernel of (dtype, head-dim tile, rows mode).
 FwdLaunchFn prefill_rows_entry(bool bf16, int dpad, int rows);
+// The half-tile kernel of (dtype, head-dim tile, rows mode).
+FwdLaunchFn half_entry(bool bf16, int dpad, int rows);
 // The key layout's kernel of (dtype, head-dim tile) for Sq = 1.
 FwdLaunchFn decode_entry(bool bf16, int dpad);
 hipError_t launch_merge(bool bf16, const MergeParams& p, hipStream_t stream);
@@ -67,6 +69,12 @@ hipError_t launch_group_merge(bool bf16, const GroupMergeParams& p, int groups, 
   template hipError_t launch_prefill<BF, DP, RM>(const FwdParams&, int, hipStream_t);
 #define FGW_MHA_EXTERN_PREFILL_ROWS(BF, DP, RM) \
   extern template hipError_t launch_prefill<BF, DP, RM>(const FwdParams&, int, hipStream_t);
+// The half-tile kernel (128 query rows), both head-dim tiles, whole and padded
+// head dims.
+#define FGW_MHA_INSTANTIATE_HALF(BF, DP, RM) \
+  template hipError_t launch_half<BF, DP, RM>(const FwdParams&, int, hipStream_t);
+#define FGW_MHA_EXTERN_HALF(BF, DP, RM) \
+  extern template hipError_t launch_half<BF, DP, RM>(const FwdParams&, int, hipStream_t);
 // The key layout's single-token kernel (Sq = 1), every head-dim tile.
 #define FGW_MHA_FOR_DECODE(X, BF) X(BF, 32) X(BF, 64) X(BF, 128) X(BF, 256)
 #define FGW_MHA_INSTANTIATE_DECODE(BF, DP) \
