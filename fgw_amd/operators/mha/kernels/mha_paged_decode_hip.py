@@ -360,17 +360,33 @@ def mha_paged_decode(q, k_cache, v_cache, block_table, cache_seqlens, page_size,
     if q.device.type != "cuda" or any(x.device != q.device or not x.is_contiguous() for x in inputs):
         raise ValueError("contiguous inputs on the same GPU required")
     capacity = block_table.shape[1] * page_size
+
+    def plan(full_kv_cache=False, cache_lengths=None):
+        return build_kernel(b, sq, h, d, k_cache.shape[0], block_table.shape[1], page_size,
+                            bool(is_causal), "float16" if q.dtype == torch.float16 else "bfloat16",
+                            q.device.index, num_splits=num_splits, split_policy=split_policy,
+                            full_kv_cache=full_kv_cache, persistent_programs=persistent_programs,
+                            cache_lengths=cache_lengths)
+
+    # A plan that no length decides (explicit splits, the legacy policy, causal
+    # calls under "auto") is made while the device still works on what the
+    # copy below waits for. What it refuses is refused after the length check.
+    kernel = None
+    if num_splits is not None or split_policy == "legacy" or (split_policy == "auto" and is_causal):
+        try:
+            kernel = plan()
+        except ValueError:
+            pass
     lengths = cache_seqlens.cpu().tolist()
-    if any(n < 0 or n > capacity for n in lengths):
+    if min(lengths) < 0 or max(lengths) > capacity:
         raise ValueError("Cache lengths must be within table capacity")
-    full_kv_cache = all(n == capacity for n in lengths)
+    if kernel is None:
+        full_kv_cache = min(lengths) == capacity
+        kernel = plan(full_kv_cache, planning_lengths(lengths, full_kv_cache, num_splits, split_policy,
+                                                      is_causal))
+    if torch.cuda.current_device() == q.device.index:
+        return kernel(*inputs)
     with torch.cuda.device(q.device):
-        kernel = build_kernel(b, sq, h, d, k_cache.shape[0], block_table.shape[1], page_size,
-                              bool(is_causal), "float16" if q.dtype == torch.float16 else "bfloat16",
-                              q.device.index, num_splits=num_splits, split_policy=split_policy,
-                              full_kv_cache=full_kv_cache, persistent_programs=persistent_programs,
-                              cache_lengths=planning_lengths(lengths, full_kv_cache, num_splits,
-                                                             split_policy, is_causal))
         return kernel(*inputs)
 
 

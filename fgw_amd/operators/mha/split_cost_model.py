@@ -53,13 +53,18 @@ def occupancy(device) -> tuple:
 
 
 def features(batch, sq, heads, dim, lengths: Sequence[int], splits, num_cus, wg_per_cu):
+    return _features(batch, sq, heads, dim, max(lengths, default=0), splits, num_cus, wg_per_cu)
+
+
+def _features(batch, sq, heads, dim, longest_length, splits, num_cus, wg_per_cu):
+    """features() of a batch whose longest cache holds longest_length keys (no
+    feature depends on the others)."""
     layout, rows, keys_round = geometry(sq, dim)
     tasks = batch * heads * math.ceil(sq / rows)
     slots = max(1, num_cus * max(1, wg_per_cu[layout]))
     items = tasks * splits
     waves = math.ceil(items / slots)
-    rounds = [math.ceil(n / keys_round) for n in lengths]
-    longest = math.ceil(max(rounds) / splits) if rounds else 0
+    longest = math.ceil(math.ceil(longest_length / keys_round) / splits)
     multi = int(splits > 1)
     parts_mb = multi * batch * heads * splits * sq * (dim + 1) * 4 * 2 / 1e6
     # Critical path in key rounds per CU: the programs resident on one CU
@@ -186,8 +191,18 @@ def balanced_split_keys(lengths, splits, capacity_tokens):
     if longest <= 0:
         return None
     budget = batch * splits
+    # The first grid value within the budget: the item count falls as the keys
+    # per split grow, so a bisection finds it (9 sums over the batch; the scan
+    # it replaces took up to 400).
     items = lambda k: sum(max(1, -(-n // k)) for n in lengths)  # noqa: E731
-    keys = next((k for k in _KEY_GRID if items(k) <= budget), None)
+    lo, hi = 0, len(_KEY_GRID)
+    while lo < hi:
+        mid = (lo + hi) // 2
+        if items(_KEY_GRID[mid]) <= budget:
+            hi = mid
+        else:
+            lo = mid + 1
+    keys = _KEY_GRID[lo] if lo < len(_KEY_GRID) else None
     rounds = lambda n: -(-n // KEYS_PER_ROUND)  # noqa: E731
     if keys is None or rounds(-(-longest // splits)) - rounds(keys) < MIN_ROUNDS_SAVED:
         return None  # the longest work item would not get shorter enough
@@ -207,10 +222,25 @@ def select_splits(batch, sq, heads, dim, capacity_tokens, lengths, device, model
         raise ValueError("No MI355X split cost model calibration is available; use split_policy='legacy'")
     if len(lengths) != batch or any(n < 0 or n > capacity_tokens for n in lengths):
         raise ValueError("cache_lengths must match batch and page-table capacity")
-    wg = occupancy(device)
-    max_split = max(1, math.ceil(capacity_tokens / 32))
-    costs = {s: predict(batch, sq, heads, dim, lengths, s, device.num_cus, wg, model)
-             for s in SPLITS if s <= max_split}
+    keys_round = geometry(sq, dim)[2]
+    return _select(batch, sq, heads, dim, -(-max(lengths, default=0) // keys_round) * keys_round,
+                   max(1, math.ceil(capacity_tokens / 32)), device.num_cus, occupancy(device),
+                   model["selection_tolerance"], model.get("absolute_margin_us", 0.0),
+                   tuple(model["weights"]))
+
+
+@lru_cache(maxsize=1024)
+def _select(batch, sq, heads, dim, longest_length, max_split, num_cus, wg, tolerance, margin, weights):
+    """select_splits for the longest cache length in whole key rounds, which is
+    all of the lengths that the features see: kept per such class, so that a
+    decode step with new lengths scores the candidates again only when its
+    longest request enters another key round (48 us of Python per call for 4
+    ragged requests with the scan of balanced_split_keys, 10 us after both)."""
+    costs = {}
+    for s in SPLITS:
+        if s <= max_split:
+            x = _features(batch, sq, heads, dim, longest_length, s, num_cus, wg)
+            costs[s] = sum(w * v for w, v in zip(weights, x))
     best = min(costs.values())
-    limit = best + max(abs(best) * model["selection_tolerance"], model.get("absolute_margin_us", 0.0))
+    limit = best + max(abs(best) * tolerance, margin)
     return min(s for s, c in costs.items() if c <= limit)
