@@ -196,9 +196,12 @@ struct CMin {
   static constexpr int value = A < B ? A : B;
 };
 
-template <bool BF16_, int DPAD_, int LAYOUT_, int STAGES_ = 0>
+// GROUPS (key layout): the page table is resolved per DMA instruction instead of
+// per block (GroupRows).
+template <bool BF16_, int DPAD_, int LAYOUT_, int STAGES_ = 0, bool GROUPS_ = false>
 struct Cfg {
   static constexpr bool BF16 = BF16_;
+  static constexpr bool GROUPS = GROUPS_;
   static constexpr int DPAD = DPAD_;  // head dim padded to a power of two >= 32
   static constexpr int LAYOUT = LAYOUT_;
   static constexpr int NWQ = LAYOUT == kLayoutQuery ? 4 : 1;  // waves along queries
@@ -242,6 +245,7 @@ struct Cfg {
   static_assert(TILE_BYTES % 1024 == 0 && INSTR % NWQ == 0 && 64 % CPR == 0, "DMA granularity");
   static_assert(NBUF == 1 || NBUF == 2, "one or two K/V stages per key group");
   static_assert(LDS_BYTES <= kLdsBudget, "LDS budget of one CU");
+  static_assert(!GROUPS || LAYOUT == kLayoutKey, "row groups: the key layout");
 };
 
 // LDS DMA (global_load_lds_dwordx4) for kernels that place their own waits
@@ -412,6 +416,67 @@ __device__ __forceinline__ void issue_tile(const FwdParams& p, const DmaLanes<C>
     const int c = IS_V ? pos_in_row ^ (4 * (r % C::VSW)) : pos_in_row ^ (r % C::KSW);
     const char* src = live && c * 8 < dim ? base + row * row_bytes + c * 16 : zero;
     __builtin_amdgcn_global_load_lds(src, FGW_LDS(void, (uintptr_t)(dst + 1024u * i)), 16, 0, 0);
+  }
+}
+
+// Row groups of the key layout (Cfg::GROUPS): page_size is a multiple of the RPI
+// key rows of one DMA instruction, so every instruction's rows lie in one page.
+// Lane i (mod INSTR) resolves instruction i of a block from a page id read one
+// block ahead; the instructions then take a uniform row base each. With a
+// table read per lane and instruction instead (issue_tile's per-key path), each
+// tile's DMA waited for its table reads and those for the DMA before them.
+template <class C>
+__device__ __forceinline__ int32_t group_id(const FwdParams& p, const int32_t* table_b, int pos0,
+                                            int lane) {
+  const u32 pg = div_page((u32)pos0 + (u32)(lane % C::INSTR * C::RPI), p.page_magic, p.page_shift);
+  const u32 last = (u32)p.width - 1u;
+  return table_b[pg < last ? pg : last];  // ids past the live pages are not used
+}
+
+// Instruction lane % INSTR of the block at pos0: pool byte offset of its first
+// row and its live rows (below len, inside the pool).
+struct GroupRows {
+  int64_t off;
+  int live;
+};
+template <class C>
+__device__ __forceinline__ GroupRows group_rows(const FwdParams& p, int64_t row_bytes, int pos0,
+                                                int32_t id, int len, int lane) {
+  const int pos = pos0 + lane % C::INSTR * C::RPI;
+  const u32 pg = div_page((u32)pos, p.page_magic, p.page_shift);
+  const int64_t row = (int64_t)id * p.page_size + ((u32)pos - pg * (u32)p.page_size);
+  const int below = len - pos < C::RPI ? len - pos : C::RPI;
+  const bool ok = below > 0 && row >= 0 && row < p.pool_rows;
+  return GroupRows{ok ? row * row_bytes : 0, ok ? below : 0};
+}
+
+// The DMA of the K and V tiles of one block from its row groups. Lanes of dead
+// rows and of chunks past D read the zero chunk. NT: non-temporal.
+template <class C, bool NT>
+__device__ __forceinline__ void issue_groups(const FwdParams& p, const DmaLanes<C>& dl,
+                                             const char* kb, const char* vb, const GroupRows& g,
+                                             unsigned char* stage, int lane) {
+  const u32 dst = (u32)opaque_uniform((int)lds_address(stage));
+  const bool full_dim = p.dim == C::DPAD;
+#pragma unroll
+  for (int q = 0; q < C::INSTR_PER_WAVE; ++q) {
+    const u32 lo = __builtin_amdgcn_readlane((u32)g.off, q);
+    const u32 hi = __builtin_amdgcn_readlane((u32)((uint64_t)g.off >> 32), q);
+    const int64_t off = (int64_t)(((uint64_t)hi << 32) | lo);
+    const int live = __builtin_amdgcn_readlane(g.live, q);
+    const u32 kd = dst + 1024u * q, vd = kd + C::TILE_BYTES;
+    const u32 ko = dl.kq(q, 0), vo = dl.vq(q, 0);
+    if (live == C::RPI && full_dim) {  // uniform
+      __builtin_amdgcn_global_load_lds(kb + off + ko, FGW_LDS(void, (uintptr_t)kd), 16, 0, NT ? 2 : 0);
+      __builtin_amdgcn_global_load_lds(vb + off + vo, FGW_LDS(void, (uintptr_t)vd), 16, 0, NT ? 2 : 0);
+    } else {
+      const char* zero = reinterpret_cast<const char*>(kZeroChunk);
+      const bool row = lane / C::CPR < live;
+      const char* ks = row && ko - dl.row_off < 2u * (u32)p.dim ? kb + off + ko : zero;
+      const char* vs = row && vo - dl.row_off < 2u * (u32)p.dim ? vb + off + vo : zero;
+      __builtin_amdgcn_global_load_lds(ks, FGW_LDS(void, (uintptr_t)kd), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(vs, FGW_LDS(void, (uintptr_t)vd), 16, 0, 0);
+    }
   }
 }
 
@@ -1202,11 +1267,18 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
     constexpr int kStep = C::NWK * C::BN;
     int spec_pos = -1;
     int32_t spec0 = 0, spec1 = 0;
+    // The page id (row groups: ids) of the block at pos.
+    auto ids_of = [&](int pos) -> int32_t {
+      if constexpr (C::GROUPS)
+        return group_id<C>(p, table_b, pos, lane);
+      else
+        return page_id(p, table_b, pos);
+    };
     if (p.mode != 2 && !p.causal && !balanced) {
       const int nfull = (capacity + C::BN - 1) / C::BN;
       spec_pos = (split_bound(nfull, split, p.splits) + wk) * C::BN;
-      if (spec_pos < capacity) spec0 = page_id(p, table_b, spec_pos);
-      if (spec_pos + kStep < capacity) spec1 = page_id(p, table_b, spec_pos + kStep);
+      if (spec_pos < capacity) spec0 = ids_of(spec_pos);
+      if (spec_pos + kStep < capacity) spec1 = ids_of(spec_pos + kStep);
     }
     int len = lengths[b];
     len = len < 0 ? 0 : (len > capacity ? capacity : len);
@@ -1248,14 +1320,23 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
     // Every key group streams its blocks n = 0, 1, ... at key
     // (blk_begin + wk + NWK n) * BN through its own LDS stages; the DMA of
     // block n + 1 is in flight while block n is computed.
-    int32_t next_id = my_n > 1 ? (spec ? spec1 : page_id(p, table_b, first_pos + kStep)) : 0;
-    if (my_n > 0) {
-      const int32_t id0 = spec ? spec0 : page_id(p, table_b, first_pos);
-      issue_tile<C, false>(p, dl, table_b, kb, row_bytes, first_pos, id0, len, group_base, wq,
-                           lane);
-      issue_tile<C, true>(p, dl, table_b, vb, row_bytes, first_pos, id0, len,
-                          group_base + C::TILE_BYTES, wq, lane);
-    }
+    int32_t next_id = my_n > 1 ? (spec ? spec1 : ids_of(first_pos + kStep)) : 0;
+    const bool nt = C::GROUPS && non_temporal_kv(p, len, row_bytes);
+    // K and V of the block at pos (its page ids: id) into a stage.
+    auto issue = [&](int pos, int32_t id, unsigned char* stage) {
+      if constexpr (C::GROUPS) {
+        const GroupRows g = group_rows<C>(p, row_bytes, pos, id, len, lane);
+        if (nt)
+          issue_groups<C, true>(p, dl, kb, vb, g, stage, lane);
+        else
+          issue_groups<C, false>(p, dl, kb, vb, g, stage, lane);
+      } else {
+        issue_tile<C, false>(p, dl, table_b, kb, row_bytes, pos, id, len, stage, wq, lane);
+        issue_tile<C, true>(p, dl, table_b, vb, row_bytes, pos, id, len, stage + C::TILE_BYTES, wq,
+                            lane);
+      }
+    };
+    if (my_n > 0) issue(first_pos, spec ? spec0 : ids_of(first_pos), group_base);
     // Q after the first DMA: its loads overlap the tile's.
     u32x4 qf[C::KK];
     {
@@ -1276,14 +1357,9 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
       wait_dma();
       group_sync<C>();  // stage n is in LDS; everyone is done with stage n - 1
       const int32_t id1 = next_id;
-      if (n + 2 < my_n) next_id = page_id(p, table_b, pos0 + 2 * kStep);
-      if (n + 1 < my_n && C::NBUF == 2) {
-        unsigned char* next = group_base + ((n + 1) % C::NBUF) * C::STAGE_BYTES;
-        issue_tile<C, false>(p, dl, table_b, kb, row_bytes, pos0 + kStep, id1, len, next, wq,
-                             lane);
-        issue_tile<C, true>(p, dl, table_b, vb, row_bytes, pos0 + kStep, id1, len,
-                            next + C::TILE_BYTES, wq, lane);
-      }
+      if (n + 2 < my_n) next_id = ids_of(pos0 + 2 * kStep);
+      if (n + 1 < my_n && C::NBUF == 2)
+        issue(pos0 + kStep, id1, group_base + ((n + 1) % C::NBUF) * C::STAGE_BYTES);
       f32x16 s[C::ST];
       u32x4 pf[C::KS];
       qk_block<C>(stage, ln, qf, s);
@@ -1292,10 +1368,7 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
       pv_block<C>(stage + C::TILE_BYTES, ln, pf, o);
       if (n + 1 < my_n && C::NBUF == 1) {
         group_sync<C>();  // single stage: refill only after every wave has read it
-        issue_tile<C, false>(p, dl, table_b, kb, row_bytes, pos0 + kStep, id1, len, stage, wq,
-                             lane);
-        issue_tile<C, true>(p, dl, table_b, vb, row_bytes, pos0 + kStep, id1, len,
-                            stage + C::TILE_BYTES, wq, lane);
+        issue(pos0 + kStep, id1, stage);
       }
     }
 
@@ -1408,9 +1481,9 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
   }
 }
 
-template <bool BF16, int DPAD, int LAYOUT, int STAGES = 0>
+template <bool BF16, int DPAD, int LAYOUT, int STAGES = 0, bool GROUPS = false>
 hipError_t launch_fwd(const FwdParams& p, int grid, hipStream_t stream) {
-  using C = Cfg<BF16, DPAD, LAYOUT, STAGES>;
+  using C = Cfg<BF16, DPAD, LAYOUT, STAGES, GROUPS>;
   fwd_kernel<C><<<dim3(grid), dim3(C::THREADS), 0, stream>>>(p, p.table, p.lengths);
   return hipGetLastError();
 }
