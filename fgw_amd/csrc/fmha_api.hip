@@ -33,8 +33,8 @@ FGW_MHA_FOR_PREFILL_ROWS(FGW_MHA_EXTERN_PREFILL_ROWS, true)
 FGW_MHA_FOR_PREFILL_ROWS(FGW_MHA_EXTERN_PREFILL_ROWS, false)
 FGW_MHA_FOR_PREFILL_ROWS(FGW_MHA_EXTERN_HALF, true)
 FGW_MHA_FOR_PREFILL_ROWS(FGW_MHA_EXTERN_HALF, false)
-FGW_MHA_FOR_KEY_GROUPS(FGW_MHA_EXTERN_KEY_GROUPS, true)
-FGW_MHA_FOR_KEY_GROUPS(FGW_MHA_EXTERN_KEY_GROUPS, false)
+FGW_MHA_FOR_GROUPS(FGW_MHA_EXTERN_GROUPS, true)
+FGW_MHA_FOR_GROUPS(FGW_MHA_EXTERN_GROUPS, false)
 FGW_MHA_FOR_DECODE(FGW_MHA_EXTERN_DECODE, true)
 FGW_MHA_FOR_DECODE(FGW_MHA_EXTERN_DECODE, false)
 
@@ -69,11 +69,12 @@ FwdLaunchFn prefill_rows_entry(bool bf16, int dpad, int rows) {
   return nullptr;
 }
 
-FwdLaunchFn key_groups_entry(bool bf16, int dpad, int stages) {
-#define FGW_KEY_GROUPS_ENTRY(BF, DP, ST) \
-  if (bf16 == BF && dpad == DP && stages == ST) return &launch_fwd<BF, DP, kLayoutKey, ST, true>;
-  FGW_MHA_FOR_KEY_GROUPS(FGW_KEY_GROUPS_ENTRY, true)
-  FGW_MHA_FOR_KEY_GROUPS(FGW_KEY_GROUPS_ENTRY, false)
+FwdLaunchFn groups_entry(bool bf16, int dpad, int layout, int stages) {
+#define FGW_GROUPS_ENTRY(BF, DP, LY, ST)                               \
+  if (bf16 == BF && dpad == DP && layout == LY && stages == ST)        \
+    return &launch_fwd<BF, DP, LY, ST, true>;
+  FGW_MHA_FOR_GROUPS(FGW_GROUPS_ENTRY, true)
+  FGW_MHA_FOR_GROUPS(FGW_GROUPS_ENTRY, false)
   return nullptr;
 }
 
@@ -511,10 +512,11 @@ int check_schedule(const fgw_mha_shape* s, const fgw_mha_schedule* sc) {
 
 // The kernel of a plan: the layout's own (`fallback`) or one of its variants.
 // - Key layout, Sq = 1: the single-token kernel where decode_takes it.
-// - Key layout: the row-group kernel where the whole-block fast path would not
-//   hold (pages that a 32-key block straddles, or a head dim below its tile)
-//   and an instruction's rows (512 / tile of them) lie in one page, and where
-//   K/V may be large enough for its non-temporal loads (non_temporal_kv looks
+// - Key and query layouts: the row-group kernel where the whole-block fast path
+//   would not hold (pages that a block, 32 keys in the key layout and 64 in the
+//   query layout, straddles, or a head dim below its tile) and an instruction's
+//   rows (512 / tile of them) lie in one page, and in the key layout where K/V
+//   may be large enough for its non-temporal loads (non_temporal_kv looks
 //   at the lengths). Measured against the plain kernel: B4 H16 Q8 KV <= 8192
 //   causal 44.1 -> 42.5 us, with pages of 16 66.7 -> 42.2; B8 H32 Q4 KV <= 2048
 //   pages of 16 65.9 -> 39.0; B2 H8 Q16 KV 32768 54.6 -> 48.9; B16 H8 Q20 D96
@@ -530,11 +532,12 @@ FwdLaunchFn kernel_of(const fgw_mha_shape* s, const fgw_mha_plan_t* p, FwdLaunch
   if (p->layout == kLayoutKey && s->sq == 1 &&
       decode_takes(p->dim_padded, (int64_t)s->heads * s->dim * 2, s->page_size))
     f = decode_entry(bf16, p->dim_padded);
-  else if (p->layout == kLayoutKey && s->page_size % (512 / p->dim_padded) == 0 &&
-           (s->page_size % 32 || s->dim != p->dim_padded ||
-            4 * (int64_t)s->batch * s->width * s->page_size * s->heads * s->dim >= kNonTemporalBytes))
-    f = key_groups_entry(bf16, p->dim_padded,
-                         p->stages == default_stages(p->layout, p->dim_padded) ? 0 : p->stages);
+  else if (p->layout != kLayoutPrefill && s->page_size % (512 / p->dim_padded) == 0 &&
+           (s->page_size % (p->layout == kLayoutKey ? 32 : 64) || s->dim != p->dim_padded ||
+            (p->layout == kLayoutKey && 4 * (int64_t)s->batch * s->width * s->page_size * s->heads *
+                                            s->dim >= kNonTemporalBytes)))
+    f = groups_entry(bf16, p->dim_padded, p->layout,
+                     p->stages == default_stages(p->layout, p->dim_padded) ? 0 : p->stages);
   else if (p->layout == kLayoutPrefill && (s->page_size % 64 || s->dim != p->dim_padded) &&
            s->page_size % (512 / p->dim_padded) == 0)
     f = prefill_rows_entry(bf16, p->dim_padded, s->dim == p->dim_padded ? kRowsGroup : kRowsPadded);

@@ -1,0 +1,7 @@
+// BF16 instantiations of the key and query layouts' row-group kernels.
+#include "fmha_kernel.h"
+#include "fmha_registry.h"
+
+namespace fgw_mha {
+FGW_MHA_FOR_GROUPS(FGW_MHA_INSTANTIATE_GROUPS, true)
+}  // namespace fgw_mha

@@ -1,0 +1,7 @@
+// F16 instantiations of the key and query layouts' row-group kernels.
+#include "fmha_kernel.h"
+#include "fmha_registry.h"
+
+namespace fgw_mha {
+FGW_MHA_FOR_GROUPS(FGW_MHA_INSTANTIATE_GROUPS, false)
+}  // namespace fgw_mha

@@ -171,7 +171,7 @@ __device__ __forceinline__ ProgramItems key_items(int work) {
   return ProgramItems{a + local, nx, local < end - a ? (end - a - local + nx - 1) / nx : 0};
 }
 
-// Whether a work item of the key layout loads K/V non-temporally: nothing
+// Whether a work item (key and query layouts) loads K/V non-temporally: nothing
 // else of the call reads its rows again (one query tile, and head rows that
 // fill whole 128-byte lines, which heads would otherwise share), and a batch
 // of requests of its length is too large for the 256 MB last-level cache to
@@ -196,8 +196,8 @@ struct CMin {
   static constexpr int value = A < B ? A : B;
 };
 
-// GROUPS (key layout): the page table is resolved per DMA instruction instead of
-// per block (GroupRows).
+// GROUPS: the page table is resolved per DMA instruction instead of per block
+// (GroupRows).
 template <bool BF16_, int DPAD_, int LAYOUT_, int STAGES_ = 0, bool GROUPS_ = false>
 struct Cfg {
   static constexpr bool BF16 = BF16_;
@@ -245,7 +245,6 @@ struct Cfg {
   static_assert(TILE_BYTES % 1024 == 0 && INSTR % NWQ == 0 && 64 % CPR == 0, "DMA granularity");
   static_assert(NBUF == 1 || NBUF == 2, "one or two K/V stages per key group");
   static_assert(LDS_BYTES <= kLdsBudget, "LDS budget of one CU");
-  static_assert(!GROUPS || LAYOUT == kLayoutKey, "row groups: the key layout");
 };
 
 // LDS DMA (global_load_lds_dwordx4) for kernels that place their own waits
@@ -419,30 +418,34 @@ __device__ __forceinline__ void issue_tile(const FwdParams& p, const DmaLanes<C>
   }
 }
 
-// Row groups of the key layout (Cfg::GROUPS): page_size is a multiple of the RPI
-// key rows of one DMA instruction, so every instruction's rows lie in one page.
-// Lane i (mod INSTR) resolves instruction i of a block from a page id read one
-// block ahead; the instructions then take a uniform row base each. With a
+// Row groups (Cfg::GROUPS): page_size is a multiple of the RPI key rows of one
+// DMA instruction, so every instruction's rows lie in one page. Lane q (mod
+// INSTR_PER_WAVE) resolves the wave's instruction q of a block from a page id
+// read one block ahead; the instructions then take a uniform row base each. With a
 // table read per lane and instruction instead (issue_tile's per-key path), each
 // tile's DMA waited for its table reads and those for the DMA before them.
 template <class C>
+__device__ __forceinline__ int group_first_row(int wq, int lane) {
+  return C::RPI * (lane % C::INSTR_PER_WAVE * C::NWQ + wq);
+}
+template <class C>
 __device__ __forceinline__ int32_t group_id(const FwdParams& p, const int32_t* table_b, int pos0,
-                                            int lane) {
-  const u32 pg = div_page((u32)pos0 + (u32)(lane % C::INSTR * C::RPI), p.page_magic, p.page_shift);
+                                            int wq, int lane) {
+  const u32 pg = div_page((u32)pos0 + (u32)group_first_row<C>(wq, lane), p.page_magic, p.page_shift);
   const u32 last = (u32)p.width - 1u;
   return table_b[pg < last ? pg : last];  // ids past the live pages are not used
 }
 
-// Instruction lane % INSTR of the block at pos0: pool byte offset of its first
-// row and its live rows (below len, inside the pool).
+// The wave's instruction lane % INSTR_PER_WAVE of the block at pos0: pool byte
+// offset of its first row and its live rows (below len, inside the pool).
 struct GroupRows {
   int64_t off;
   int live;
 };
 template <class C>
 __device__ __forceinline__ GroupRows group_rows(const FwdParams& p, int64_t row_bytes, int pos0,
-                                                int32_t id, int len, int lane) {
-  const int pos = pos0 + lane % C::INSTR * C::RPI;
+                                                int32_t id, int len, int wq, int lane) {
+  const int pos = pos0 + group_first_row<C>(wq, lane);
   const u32 pg = div_page((u32)pos, p.page_magic, p.page_shift);
   const int64_t row = (int64_t)id * p.page_size + ((u32)pos - pg * (u32)p.page_size);
   const int below = len - pos < C::RPI ? len - pos : C::RPI;
@@ -455,7 +458,7 @@ __device__ __forceinline__ GroupRows group_rows(const FwdParams& p, int64_t row_
 template <class C, bool NT>
 __device__ __forceinline__ void issue_groups(const FwdParams& p, const DmaLanes<C>& dl,
                                              const char* kb, const char* vb, const GroupRows& g,
-                                             unsigned char* stage, int lane) {
+                                             unsigned char* stage, int wq, int lane) {
   const u32 dst = (u32)opaque_uniform((int)lds_address(stage));
   const bool full_dim = p.dim == C::DPAD;
 #pragma unroll
@@ -464,8 +467,8 @@ __device__ __forceinline__ void issue_groups(const FwdParams& p, const DmaLanes<
     const u32 hi = __builtin_amdgcn_readlane((u32)((uint64_t)g.off >> 32), q);
     const int64_t off = (int64_t)(((uint64_t)hi << 32) | lo);
     const int live = __builtin_amdgcn_readlane(g.live, q);
-    const u32 kd = dst + 1024u * q, vd = kd + C::TILE_BYTES;
-    const u32 ko = dl.kq(q, 0), vo = dl.vq(q, 0);
+    const u32 kd = dst + 1024u * (u32)(q * C::NWQ + wq), vd = kd + C::TILE_BYTES;
+    const u32 ko = dl.kq(q, wq), vo = dl.vq(q, wq);
     if (live == C::RPI && full_dim) {  // uniform
       __builtin_amdgcn_global_load_lds(kb + off + ko, FGW_LDS(void, (uintptr_t)kd), 16, 0, NT ? 2 : 0);
       __builtin_amdgcn_global_load_lds(vb + off + vo, FGW_LDS(void, (uintptr_t)vd), 16, 0, NT ? 2 : 0);
@@ -1270,7 +1273,7 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
     // The page id (row groups: ids) of the block at pos.
     auto ids_of = [&](int pos) -> int32_t {
       if constexpr (C::GROUPS)
-        return group_id<C>(p, table_b, pos, lane);
+        return group_id<C>(p, table_b, pos, wq, lane);
       else
         return page_id(p, table_b, pos);
     };
@@ -1325,11 +1328,11 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
     // K and V of the block at pos (its page ids: id) into a stage.
     auto issue = [&](int pos, int32_t id, unsigned char* stage) {
       if constexpr (C::GROUPS) {
-        const GroupRows g = group_rows<C>(p, row_bytes, pos, id, len, lane);
+        const GroupRows g = group_rows<C>(p, row_bytes, pos, id, len, wq, lane);
         if (nt)
-          issue_groups<C, true>(p, dl, kb, vb, g, stage, lane);
+          issue_groups<C, true>(p, dl, kb, vb, g, stage, wq, lane);
         else
-          issue_groups<C, false>(p, dl, kb, vb, g, stage, lane);
+          issue_groups<C, false>(p, dl, kb, vb, g, stage, wq, lane);
       } else {
         issue_tile<C, false>(p, dl, table_b, kb, row_bytes, pos, id, len, stage, wq, lane);
         issue_tile<C, true>(p, dl, table_b, vb, row_bytes, pos, id, len, stage + C::TILE_BYTES, wq,

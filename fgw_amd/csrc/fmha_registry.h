@@ -27,8 +27,8 @@ inline int dim_tile(int dim) {
 FwdEntry fwd_entry(bool bf16, int dpad, int layout, int stages = 0);
 // The prefill layout's row-group kernel of (dtype, head-dim tile, rows mode).
 FwdLaunchFn prefill_rows_entry(bool bf16, int dpad, int rows);
-// The key layout's row-group kernel of (dtype, head-dim tile, stages).
-FwdLaunchFn key_groups_entry(bool bf16, int dpad, int stages);
+// The row-group kernel of (dtype, head-dim tile, key or query layout, stages).
+FwdLaunchFn groups_entry(bool bf16, int dpad, int layout, int stages);
 // The half-tile kernel of (dtype, head-dim tile, rows mode).
 FwdLaunchFn half_entry(bool bf16, int dpad, int rows);
 // The key layout's kernel of (dtype, head-dim tile) for Sq = 1.
@@ -71,13 +71,16 @@ hipError_t launch_group_merge(bool bf16, const GroupMergeParams& p, int groups, 
   template hipError_t launch_prefill<BF, DP, RM>(const FwdParams&, int, hipStream_t);
 #define FGW_MHA_EXTERN_PREFILL_ROWS(BF, DP, RM) \
   extern template hipError_t launch_prefill<BF, DP, RM>(const FwdParams&, int, hipStream_t);
-// The key layout's row-group kernels: every head-dim tile, and the
-// single-stage variant of tile 128.
-#define FGW_MHA_FOR_KEY_GROUPS(X, BF) X(BF, 32, 0) X(BF, 64, 0) X(BF, 128, 0) X(BF, 256, 0) X(BF, 128, 1)
-#define FGW_MHA_INSTANTIATE_KEY_GROUPS(BF, DP, ST) \
-  template hipError_t launch_fwd<BF, DP, kLayoutKey, ST, true>(const FwdParams&, int, hipStream_t);
-#define FGW_MHA_EXTERN_KEY_GROUPS(BF, DP, ST) \
-  extern template hipError_t launch_fwd<BF, DP, kLayoutKey, ST, true>(const FwdParams&, int, hipStream_t);
+// The row-group kernels of the key layout (every head-dim tile, and the
+// single-stage variant of tile 128) and of the query layout.
+#define FGW_MHA_FOR_GROUPS(X, BF)                                                              \
+  X(BF, 32, kLayoutKey, 0) X(BF, 64, kLayoutKey, 0) X(BF, 128, kLayoutKey, 0)                  \
+  X(BF, 256, kLayoutKey, 0) X(BF, 128, kLayoutKey, 1) X(BF, 32, kLayoutQuery, 0)               \
+  X(BF, 64, kLayoutQuery, 0) X(BF, 128, kLayoutQuery, 0) X(BF, 256, kLayoutQuery, 0)
+#define FGW_MHA_INSTANTIATE_GROUPS(BF, DP, LY, ST) \
+  template hipError_t launch_fwd<BF, DP, LY, ST, true>(const FwdParams&, int, hipStream_t);
+#define FGW_MHA_EXTERN_GROUPS(BF, DP, LY, ST) \
+  extern template hipError_t launch_fwd<BF, DP, LY, ST, true>(const FwdParams&, int, hipStream_t);
 // The half-tile kernel (128 query rows), both head-dim tiles, whole and padded
 // head dims.
 #define FGW_MHA_INSTANTIATE_HALF(BF, DP, RM) \

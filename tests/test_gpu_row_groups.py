@@ -1,4 +1,4 @@
-"""The key layout's row-group kernels (Sq > 1) against the oracle.
+"""The row-group kernels of the key layout (Sq > 1) and the query layout against the oracle.
 
 Where they can go wrong: caches that end inside an instruction's rows or a
 block, pages of one instruction's rows and off the powers of two (odd sizes
@@ -16,7 +16,7 @@ from oracle import mha_oracle as O
 gpu = pytest.mark.gpu
 
 
-def _check(b, sq, h, d, page, lengths, dtype, causal=False, outside=False, **plan):
+def _check(b, sq, h, d, page, lengths, dtype, causal=False, outside=False, layout="key", **plan):
     from fgw_amd.operators.mha.current import build_kernel
     width = -(-max(lengths) // page)
     q, k, v, table = O.make_inputs(("groups", b, sq, h, d, page, width), 17, dtype)
@@ -31,7 +31,7 @@ def _check(b, sq, h, d, page, lengths, dtype, causal=False, outside=False, **pla
         etable = table.clone()
         etable[0, 0] = etable[-1, 1] = k.shape[0] // page
     kern = build_kernel(b, sq, h, d, k.shape[0], width, page, causal,
-                        "float16" if dtype == torch.float16 else "bfloat16", 0, layout="key", **plan)
+                        "float16" if dtype == torch.float16 else "bfloat16", 0, layout=layout, **plan)
     got = kern(*[x.cuda() for x in (q, k, v, table, lengths)]).cpu()
     rtol, atol = O.TOLERANCES[dtype]
     torch.testing.assert_close(got, O.chunked_reference(q, ek, ev, etable, lengths, page, causal),
@@ -66,3 +66,23 @@ def test_length_balanced_and_non_temporal():
            split_keys=128)
     # 2 x 40 x 4096 x 8 x 64 x 2 bytes = 168 MB of K/V.
     _check(40, 2, 8, 64, 128, [4096 - 31 * i for i in range(40)], torch.float16, num_splits=1)
+
+
+@gpu
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d,page,dtype", [
+    (16, 16, torch.bfloat16), (32, 48, torch.float16), (48, 8, torch.bfloat16),
+    (64, 32, torch.float16), (96, 64, torch.float16), (128, 16, torch.bfloat16),
+    (192, 2, torch.bfloat16), (192, 64, torch.float16), (256, 16, torch.float16)])
+def test_query_layout_ragged_ends(d, page, dtype, causal):
+    lengths = [0, 1, 3, 63, 64, 65, 130, 257, 300, 520]
+    for sq, splits in ((33, 1), (129, 2)):
+        _check(len(lengths), sq, 2, d, page, lengths, dtype, causal, layout="query",
+               num_splits=splits)
+
+
+@gpu
+def test_query_layout_ids_outside_the_pool_and_several_items():
+    _check(2, 150, 3, 256, 32, [400, 177], torch.bfloat16, outside=True, layout="query", num_splits=1,
+           persistent_programs=4)
+    _check(2, 150, 3, 192, 64, [400, 177], torch.float16, outside=True, layout="query", num_splits=2)
