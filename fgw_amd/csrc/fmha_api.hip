@@ -731,7 +731,18 @@ int fgw_mha_plan(const fgw_mha_shape* s, const fgw_mha_request* req,
     // doubling past them makes a second wave of items (B1H1 Q3712/KV4096:
     // 15 tiles x 32 splits = 480 items on 256 slots, 55.8 us, against 31.2 us
     // at 16 splits).
-    const int64_t slots = (int64_t)dev->num_cus * wg_default;
+    // The query layout's head-dim tile 256 fills a CU's LDS with one workgroup,
+    // whatever the tile-128 kernel's occupancy (wg_default): counting two ran
+    // the items in two waves and merged twice the partials (direct time / at
+    // half the splits: B1 H8 Q512 KV 4096 causal 55.4 / 40.4 us, B1 H16 Q100 KV
+    // 8192 57.9 / 43.7, B2 H8 Q1024 KV 2048 72.4 / 59.8, causal 69.5 / 60.1).
+    // Causal tiles of very different lengths keep the finer items, which
+    // balance better (B1 H8 S2048 56.0 / 59.6, B1 H4 S4096 93.6 / 97.2).
+    int wg_fill = wg_default;
+    if (layout == kLayoutQuery && dpad == 256 &&
+        !(s->causal && 3 * (int64_t)(2 * capacity - s->sq) < 4 * capacity))
+      wg_fill = 1;
+    const int64_t slots = (int64_t)dev->num_cus * wg_fill;
     splits = 1;
     while (splits < kAutoMaxSplits && tasks * splits * 2 <= slots &&
            (int64_t)(splits * 2) * min_keys <= capacity)
