@@ -35,6 +35,8 @@ FGW_MHA_FOR_PREFILL_ROWS(FGW_MHA_EXTERN_HALF, true)
 FGW_MHA_FOR_PREFILL_ROWS(FGW_MHA_EXTERN_HALF, false)
 FGW_MHA_FOR_GROUPS(FGW_MHA_EXTERN_GROUPS, true)
 FGW_MHA_FOR_GROUPS(FGW_MHA_EXTERN_GROUPS, false)
+extern FGW_MHA_INSTANTIATE_DUAL(true)
+extern FGW_MHA_INSTANTIATE_DUAL(false)
 FGW_MHA_FOR_DECODE(FGW_MHA_EXTERN_DECODE, true)
 FGW_MHA_FOR_DECODE(FGW_MHA_EXTERN_DECODE, false)
 
@@ -72,10 +74,15 @@ FwdLaunchFn prefill_rows_entry(bool bf16, int dpad, int rows) {
 FwdLaunchFn groups_entry(bool bf16, int dpad, int layout, int stages) {
 #define FGW_GROUPS_ENTRY(BF, DP, LY, ST)                               \
   if (bf16 == BF && dpad == DP && layout == LY && stages == ST)        \
-    return &launch_fwd<BF, DP, LY, ST, true>;
+    return &launch_fwd<BF, DP, LY, ST, kGroups>;
   FGW_MHA_FOR_GROUPS(FGW_GROUPS_ENTRY, true)
   FGW_MHA_FOR_GROUPS(FGW_GROUPS_ENTRY, false)
   return nullptr;
+}
+
+FwdLaunchFn dual_entry(bool bf16) {
+  return bf16 ? &launch_fwd<true, 256, kLayoutQuery, 0, kDual>
+              : &launch_fwd<false, 256, kLayoutQuery, 0, kDual>;
 }
 
 FwdLaunchFn half_entry(bool bf16, int dpad, int rows) {
@@ -510,6 +517,23 @@ int check_schedule(const fgw_mha_shape* s, const fgw_mha_schedule* sc) {
   return FGW_MHA_OK;
 }
 
+// Whether a query-layout plan runs on the eight-wave kernel (kDual, head-dim
+// tile 256): whole 64-key blocks at D 256, and items long enough (visible keys
+// of the average row at full table capacity, per split) that a block's gain
+// outweighs the 2 us in which the two states meet. Measured, plain / eight
+// waves (three rotating sets of inputs): 64 keys per item (B2 H8 Q64) 8.6 / 10.6
+// us, 256 (B8 H32 Q128) 21.0 / 21.5, 512 (B8 H32 Q128) 33.8 / 35.8, 512 (B4 H8
+// Q200 KV <= 2048) 37.6 / 36.7, 768 (B2 H8 Q1024 KV 2048 causal) 59.8 / 55.2,
+// 1024 (B8 H32 Q64, ragged, FP16) 53.7 / 48.7, 2048 (B1 H16 S4096 causal) 197 /
+// 163, 2048 (B1 H32 Q2048, FP16) 174 / 157.
+constexpr int64_t kDualMinKeys = 768;
+bool dual_takes(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
+  const int64_t capacity = (int64_t)s->width * s->page_size;
+  const int64_t hidden = !s->causal ? 0 : (s->sq < capacity ? s->sq : capacity) / 2;
+  return p->layout == kLayoutQuery && s->dim == 256 && s->page_size % 64 == 0 &&
+         capacity - hidden >= kDualMinKeys * (p->num_splits > 1 ? p->num_splits : 1);
+}
+
 // The kernel of a plan: the layout's own (`fallback`) or one of its variants.
 // - Key layout, Sq = 1: the single-token kernel where decode_takes it.
 // - Key and query layouts: the row-group kernel where the whole-block fast path
@@ -523,6 +547,7 @@ int check_schedule(const fgw_mha_shape* s, const fgw_mha_schedule* sc) {
 //   pages of 48 21.4 -> 15.7; B8 H32 Q5 D32 pages of 16 71.5 -> 38.6. Small
 //   calls of whole blocks keep the plain kernel (B1 H8 Q4 D64 KV 512 9.35
 //   against 9.57, B2 H8 Q16 KV 2048 13.4 against 13.6).
+// - Query layout: the eight-wave kernel where dual_takes it.
 // - Prefill layout: a row-group variant where the whole-block fast path would
 //   not hold (pages that a 64-key block straddles, or a head dim below its
 //   tile) and an instruction's rows (512 / tile of them) still lie in one page.
@@ -538,6 +563,8 @@ FwdLaunchFn kernel_of(const fgw_mha_shape* s, const fgw_mha_plan_t* p, FwdLaunch
                                             s->dim >= kNonTemporalBytes)))
     f = groups_entry(bf16, p->dim_padded, p->layout,
                      p->stages == default_stages(p->layout, p->dim_padded) ? 0 : p->stages);
+  else if (dual_takes(s, p))
+    f = dual_entry(bf16);
   else if (p->layout == kLayoutPrefill && (s->page_size % 64 || s->dim != p->dim_padded) &&
            s->page_size % (512 / p->dim_padded) == 0)
     f = prefill_rows_entry(bf16, p->dim_padded, s->dim == p->dim_padded ? kRowsGroup : kRowsPadded);

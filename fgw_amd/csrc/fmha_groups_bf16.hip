@@ -1,7 +1,9 @@
-// BF16 instantiations of the key and query layouts' row-group kernels.
+// BF16 instantiations of the key and query layouts' row-group kernels and of the
+// query layout's eight-wave kernel.
 #include "fmha_kernel.h"
 #include "fmha_registry.h"
 
 namespace fgw_mha {
 FGW_MHA_FOR_GROUPS(FGW_MHA_INSTANTIATE_GROUPS, true)
+FGW_MHA_INSTANTIATE_DUAL(true)
 }  // namespace fgw_mha

@@ -1,7 +1,9 @@
-// F16 instantiations of the key and query layouts' row-group kernels.
+// F16 instantiations of the key and query layouts' row-group kernels and of the
+// query layout's eight-wave kernel.
 #include "fmha_kernel.h"
 #include "fmha_registry.h"
 
 namespace fgw_mha {
 FGW_MHA_FOR_GROUPS(FGW_MHA_INSTANTIATE_GROUPS, false)
+FGW_MHA_INSTANTIATE_DUAL(false)
 }  // namespace fgw_mha

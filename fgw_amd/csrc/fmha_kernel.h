@@ -196,17 +196,33 @@ struct CMin {
   static constexpr int value = A < B ? A : B;
 };
 
-// GROUPS: the page table is resolved per DMA instruction instead of per block
+// Variants of fwd_kernel.
+// kGroups: the page table is resolved per DMA instruction instead of per block
 // (GroupRows).
-template <bool BF16_, int DPAD_, int LAYOUT_, int STAGES_ = 0, bool GROUPS_ = false>
+// kDual (query layout, head-dim tile 256): two sets of four waves hold the same
+// 128 query rows, each takes 32 keys of every 64-key block, and their states
+// meet in LDS at the end of an item. At this tile the K/V stages fill a CU's LDS
+// with one workgroup; with four waves every SIMD had one, whose chain of LDS
+// reads, MFMAs and softmax nothing overlapped (2.6 us per block for 0.9 us of
+// MFMAs). With eight, one set's softmax runs beside the other's MFMAs, at the
+// same LDS and the same loads; what bounds it is still the chain (two waves per
+// SIMD at 256 registers). BF16, plain / eight waves: B1 H16 S4096 causal 197 / 163
+// us, B2 H8 Q1024 KV 2048 causal 59.8 / 55.2 us. Which plans take it: dual_takes
+// (fmha_api.hip). With padded head dims and small pages (row groups) the same
+// split measured 0.73 to 1.08 of the plain kernel's speed, and is not built.
+enum Variant : int { kPlain = 0, kGroups = 1, kDual = 2 };
+template <bool BF16_, int DPAD_, int LAYOUT_, int STAGES_ = 0, int VARIANT_ = kPlain>
 struct Cfg {
   static constexpr bool BF16 = BF16_;
-  static constexpr bool GROUPS = GROUPS_;
+  static constexpr int VARIANT = VARIANT_;
+  static constexpr bool GROUPS = VARIANT == kGroups;
   static constexpr int DPAD = DPAD_;  // head dim padded to a power of two >= 32
   static constexpr int LAYOUT = LAYOUT_;
   static constexpr int NWQ = LAYOUT == kLayoutQuery ? 4 : 1;  // waves along queries
-  static constexpr int NWK = LAYOUT == kLayoutQuery ? 1 : 4;  // waves along keys
-  static constexpr int BN = LAYOUT == kLayoutQuery ? 64 : 32; // keys per block
+  static constexpr bool DUAL = VARIANT == kDual;
+  static constexpr int NWK = LAYOUT == kLayoutQuery ? (DUAL ? 2 : 1) : 4;  // waves along keys
+  static constexpr int BLOCK = LAYOUT == kLayoutQuery ? 64 : 32;  // keys per block of the split partition
+  static constexpr int BN = DUAL ? BLOCK / 2 : BLOCK;             // keys per tile
   static constexpr int WAVES = NWQ * NWK;
   static constexpr int THREADS = 64 * WAVES;
   static constexpr int ROWS_WAVE = 32;
@@ -225,7 +241,8 @@ struct Cfg {
   static constexpr int TILES_BYTES = NWK * GROUP_BYTES;
   static constexpr int OSTRIDE = DPAD + 4;  // combine buffer row stride (floats)
   static constexpr int COMB_BYTES =
-      NWK > 1 ? (2 * NWK * ROWS_WAVE + NWK * ROWS_WAVE * OSTRIDE) * 4 : 0;
+      DUAL ? NWQ * (DT * 4096 + 512)
+      : NWK > 1 ? (2 * NWK * ROWS_WAVE + NWK * ROWS_WAVE * OSTRIDE) * 4 : 0;
   // Key layout: per-request split prefix sums of a length-balanced plan,
   // after the tiles and the combine buffer.
   static constexpr int PREFIX_OFF = CMax<TILES_BYTES, COMB_BYTES>::value;
@@ -240,7 +257,7 @@ struct Cfg {
   static constexpr int KSW = CMin<16, CPR>::value;  // K: x = r % KSW
   static constexpr int VSW = CPR / 4;               // V: x = 4 * (r % VSW)
   static constexpr int RPI = 64 / CPR;              // key rows per DMA instruction
-  static_assert(NWQ == 1 || NWK == 1, "tiles are shared by all waves or by none");
+  static_assert(NWQ == 1 || NWK == 1 || DUAL, "tiles are shared by all waves, by none or by halves");
   static_assert((DPAD & (DPAD - 1)) == 0 && DPAD >= 32 && DPAD <= 256, "head dim tile");
   static_assert(TILE_BYTES % 1024 == 0 && INSTR % NWQ == 0 && 64 % CPR == 0, "DMA granularity");
   static_assert(NBUF == 1 || NBUF == 2, "one or two K/V stages per key group");
@@ -253,7 +270,8 @@ struct Cfg {
 // for every outstanding DMA before each transposing LDS read), and the
 // kernels wait for them explicitly with wait_vm. The compiler's own vmcnt
 // waits stay correct: loads retire in order, so extra loads it does not know
-// of can only make its waits stricter. fwd_kernel uses the compiler builtin.
+// of can only make its waits stricter. fwd_kernel uses the compiler builtin, but
+// for kDual.
 // Byte address of a shared-memory pointer within the workgroup's LDS.
 __device__ __forceinline__ u32 lds_address(const void* p) {
   return (u32)(uintptr_t)FGW_LDS(const void, p);
@@ -389,8 +407,13 @@ __device__ __forceinline__ void issue_tile(const FwdParams& p, const DmaLanes<C>
       const int i = q * C::NWQ + wq;
       const int64_t rb = (row0 + C::RPI * i) * row_bytes;
       const u32 off = IS_V ? dl.vq(q, wq) : dl.kq(q, wq);
-      __builtin_amdgcn_global_load_lds(base + rb + off, FGW_LDS(void, (uintptr_t)(dst + 1024u * i)),
-                                       16, 0, 0);
+      // With the builtin the compiler waits for all DMA in flight before the
+      // transposing reads of V; kDual's waits are its own (fwd_kernel's loop).
+      if constexpr (C::DUAL)
+        dma_saddr(base + rb, off, dst + 1024u * i);
+      else
+        __builtin_amdgcn_global_load_lds(base + rb + off,
+                                         FGW_LDS(void, (uintptr_t)(dst + 1024u * i)), 16, 0, 0);
     }
     return;
   }
@@ -414,11 +437,14 @@ __device__ __forceinline__ void issue_tile(const FwdParams& p, const DmaLanes<C>
     const bool live = pos < len && row >= 0 && row < p.pool_rows;
     const int c = IS_V ? pos_in_row ^ (4 * (r % C::VSW)) : pos_in_row ^ (r % C::KSW);
     const char* src = live && c * 8 < dim ? base + row * row_bytes + c * 16 : zero;
-    __builtin_amdgcn_global_load_lds(src, FGW_LDS(void, (uintptr_t)(dst + 1024u * i)), 16, 0, 0);
+    if constexpr (C::DUAL)
+      dma_flat(src, dst + 1024u * i);
+    else
+      __builtin_amdgcn_global_load_lds(src, FGW_LDS(void, (uintptr_t)(dst + 1024u * i)), 16, 0, 0);
   }
 }
 
-// Row groups (Cfg::GROUPS): page_size is a multiple of the RPI key rows of one
+// Row groups (kGroups): page_size is a multiple of the RPI key rows of one
 // DMA instruction, so every instruction's rows lie in one page. Lane q (mod
 // INSTR_PER_WAVE) resolves the wave's instruction q of a block from a page id
 // read one block ahead; the instructions then take a uniform row base each. With a
@@ -1188,8 +1214,8 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int il = lane & 31, hh = lane >> 5;
-  const int wq = C::NWQ > 1 ? wave : 0;
-  const int wk = C::NWK > 1 ? wave : 0;
+  const int wq = C::NWQ > 1 ? (C::DUAL ? wave % C::NWQ : wave) : 0;
+  const int wk = C::NWK > 1 ? wave / C::NWQ : 0;
   unsigned char* const group_base = smem + wk * C::GROUP_BYTES;
   const Lanes<C> ln(lane);
   const int64_t row_bytes = (int64_t)p.heads * p.dim * 2;
@@ -1268,18 +1294,20 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
     // together with the length instead of after it; a shorter length moves
     // the block range and they are read again below.
     constexpr int kStep = C::NWK * C::BN;
+    // Key of the wave's first tile of an item whose blocks start at blk.
+    auto tile_of = [&](int blk) { return C::DUAL ? blk * C::BLOCK + wk * C::BN : (blk + wk) * C::BN; };
     int spec_pos = -1;
     int32_t spec0 = 0, spec1 = 0;
     // The page id (row groups: ids) of the block at pos.
     auto ids_of = [&](int pos) -> int32_t {
       if constexpr (C::GROUPS)
         return group_id<C>(p, table_b, pos, wq, lane);
-      else
-        return page_id(p, table_b, pos);
+      else  // (DUAL: the second half of the last block may lie past the table)
+        return page_id(p, table_b, C::DUAL && pos >= capacity ? 0 : pos);
     };
     if (p.mode != 2 && !p.causal && !balanced) {
-      const int nfull = (capacity + C::BN - 1) / C::BN;
-      spec_pos = (split_bound(nfull, split, p.splits) + wk) * C::BN;
+      const int nfull = (capacity + C::BLOCK - 1) / C::BLOCK;
+      spec_pos = tile_of(split_bound(nfull, split, p.splits));
       if (spec_pos < capacity) spec0 = ids_of(spec_pos);
       if (spec_pos + kStep < capacity) spec1 = ids_of(spec_pos + kStep);
     }
@@ -1289,7 +1317,7 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
     const int tile_last = (q0 + C::ROWS_TILE < p.sq ? q0 + C::ROWS_TILE : p.sq) - 1;
     int max_vis = p.causal ? len - p.sq + tile_last + 1 : len;
     max_vis = max_vis < 0 ? 0 : (max_vis > len ? len : max_vis);
-    const int nblk = (max_vis + C::BN - 1) / C::BN;
+    const int nblk = (max_vis + C::BLOCK - 1) / C::BLOCK;
     int blk_begin, blk_end;
     if (p.mode == 2) {  // the segment's blocks that hold visible keys
       blk_end = seg_hi < nblk ? seg_hi : nblk;
@@ -1299,7 +1327,8 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
       blk_end = split_bound(nblk, split + 1, nsplit);
     }
     const int cnt = blk_end - blk_begin;
-    const int my_n = cnt > wk ? (cnt - wk + C::NWK - 1) / C::NWK : 0;
+    // (DUAL: both sets take every block, so they meet at the same barriers.)
+    const int my_n = C::DUAL ? cnt : (cnt > wk ? (cnt - wk + C::NWK - 1) / C::NWK : 0);
 
     // Rows of this wave and their visible key counts; blocks that end above
     // wmin hold keys some row of the wave cannot see and are masked.
@@ -1317,7 +1346,7 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
 #pragma unroll
       for (int v = 0; v < 16; ++v) o[dt][v] = 0.0f;
 
-    const int first_pos = (blk_begin + wk) * C::BN;
+    const int first_pos = tile_of(blk_begin);
     const bool spec = first_pos == spec_pos;
     if (it > 0) __syncthreads();  // LDS of the previous work item is no longer read
     // Every key group streams its blocks n = 0, 1, ... at key
@@ -1377,12 +1406,41 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
 
     wait_dma();  // no DMA of this work item outlives it
     p = *kernarg();  // the output's parameters, not held across the main loop
-    if constexpr (C::NWK == 1) {
+    if constexpr (C::DUAL) {
+      // The second set's state to the first through LDS, lane to lane.
+      __syncthreads();  // no wave reads the tiles any more
+      f32x4* const so = reinterpret_cast<f32x4*>(smem + wq * C::DT * 4096);
+      float* const sml = reinterpret_cast<float*>(smem + C::NWQ * C::DT * 4096 + wq * 512);
+      const int lo = opaque_lane(lane);
+      if (wk == 1) {
+        sml[lo] = m;
+        sml[64 + lo] = l;
+#pragma unroll
+        for (int i = 0; i < 4 * C::DT; ++i)
+          so[i * 64 + lo] = f32x4{o[i / 4][4 * (i % 4)], o[i / 4][4 * (i % 4) + 1],
+                                  o[i / 4][4 * (i % 4) + 2], o[i / 4][4 * (i % 4) + 3]};
+      }
+      __syncthreads();
+      if (wk == 0) {
+        const float mb = sml[lo], top = fmaxf(m, mb);
+        const float wa = __builtin_amdgcn_exp2f(m - top), wb = __builtin_amdgcn_exp2f(mb - top);
+        l = l * wa + sml[64 + lo] * wb;
+        m = top;
+#pragma unroll
+        for (int i = 0; i < 4 * C::DT; ++i) {
+          const f32x4 x = so[i * 64 + lo];
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            o[i / 4][4 * (i % 4) + j] = o[i / 4][4 * (i % 4) + j] * wa + x[j] * wb;
+        }
+      }
+    }
+    if constexpr (C::NWQ > 1) {
       const float tot = pair_sum(l);
       // Direct stores: D < DPAD, or D tiles below 128 (staged, D tile 64
       // measured 1.3% slower on two query-layout shapes).
       auto store_direct = [&]() {
-        if (qrow >= p.sq) return;
+        if (qrow >= p.sq || wk > 0) return;
         const float inv = 1.0f / fmaxf(tot, 1.0e-30f);
         const int ho = opaque_lane(hh);
 #pragma unroll
@@ -1414,7 +1472,7 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
               f32 ? nullptr
                   : static_cast<unsigned char*>(p.out) +
                         (((int64_t)b * p.sq + row_base) * p.heads + h) * C::DPAD * 2;
-          store_rows_staged<C>(smem + wq * 32 * kStagedRowBytes<C>, lane, o,
+          if (wk == 0) store_rows_staged<C>(smem + wq * 32 * kStagedRowBytes<C>, lane, o,
                                1.0f / fmaxf(tot, 1.0e-30f), f32, fdst, bdst,
                                (int64_t)p.heads * C::DPAD * 2, p.sq - row_base);
         } else {
@@ -1423,7 +1481,7 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
       } else {
         store_direct();
       }
-      if (qrow < p.sq && hh == 0) {
+      if (qrow < p.sq && hh == 0 && wk == 0) {
         if (p.mode == 1)
           p.lse[(((int64_t)b * p.heads + h) * p.splits + split) * p.sq + qrow] = lse_of(m, tot);
         else if (p.mode == 2 && slot >= 0)
@@ -1484,9 +1542,9 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
   }
 }
 
-template <bool BF16, int DPAD, int LAYOUT, int STAGES = 0, bool GROUPS = false>
+template <bool BF16, int DPAD, int LAYOUT, int STAGES = 0, int VARIANT = kPlain>
 hipError_t launch_fwd(const FwdParams& p, int grid, hipStream_t stream) {
-  using C = Cfg<BF16, DPAD, LAYOUT, STAGES, GROUPS>;
+  using C = Cfg<BF16, DPAD, LAYOUT, STAGES, VARIANT>;
   fwd_kernel<C><<<dim3(grid), dim3(C::THREADS), 0, stream>>>(p, p.table, p.lengths);
   return hipGetLastError();
 }

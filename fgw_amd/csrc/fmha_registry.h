@@ -29,6 +29,8 @@ FwdEntry fwd_entry(bool bf16, int dpad, int layout, int stages = 0);
 FwdLaunchFn prefill_rows_entry(bool bf16, int dpad, int rows);
 // The row-group kernel of (dtype, head-dim tile, key or query layout, stages).
 FwdLaunchFn groups_entry(bool bf16, int dpad, int layout, int stages);
+// The query layout's kernel of eight waves (kDual), head-dim tile 256.
+FwdLaunchFn dual_entry(bool bf16);
 // The half-tile kernel of (dtype, head-dim tile, rows mode).
 FwdLaunchFn half_entry(bool bf16, int dpad, int rows);
 // The key layout's kernel of (dtype, head-dim tile) for Sq = 1.
@@ -78,9 +80,12 @@ hipError_t launch_group_merge(bool bf16, const GroupMergeParams& p, int groups, 
   X(BF, 256, kLayoutKey, 0) X(BF, 128, kLayoutKey, 1) X(BF, 32, kLayoutQuery, 0)               \
   X(BF, 64, kLayoutQuery, 0) X(BF, 128, kLayoutQuery, 0) X(BF, 256, kLayoutQuery, 0)
 #define FGW_MHA_INSTANTIATE_GROUPS(BF, DP, LY, ST) \
-  template hipError_t launch_fwd<BF, DP, LY, ST, true>(const FwdParams&, int, hipStream_t);
+  template hipError_t launch_fwd<BF, DP, LY, ST, kGroups>(const FwdParams&, int, hipStream_t);
 #define FGW_MHA_EXTERN_GROUPS(BF, DP, LY, ST) \
-  extern template hipError_t launch_fwd<BF, DP, LY, ST, true>(const FwdParams&, int, hipStream_t);
+  extern template hipError_t launch_fwd<BF, DP, LY, ST, kGroups>(const FwdParams&, int, hipStream_t);
+// The query layout's eight-wave kernel, head-dim tile 256.
+#define FGW_MHA_INSTANTIATE_DUAL(BF) \
+  template hipError_t launch_fwd<BF, 256, kLayoutQuery, 0, kDual>(const FwdParams&, int, hipStream_t);
 // The half-tile kernel (128 query rows), both head-dim tiles, whole and padded
 // head dims.
 #define FGW_MHA_INSTANTIATE_HALF(BF, DP, RM) \
