@@ -180,7 +180,11 @@ __device__ __forceinline__ ProgramItems key_items(int work) {
 // Measured over three rotating sets of inputs, the time non-temporal over
 // plain: B8 H8 D128 KV 512 / 1024 / 2048 (16 / 32 / 64 MiB) 1.20 / 1.29 /
 // 1.07, KV 3072 (96 MiB) 0.99, KV 4096-8192 (128-256 MiB) 0.89-0.90; D 16 and
-// 48 (shared lines) 1.45 and 1.11; two query tiles 1.21.
+// 48 (shared lines) 1.45 and 1.11; two query tiles 1.21. The price: a program that
+// repeats one call on one set of 128-256 MiB, with nothing in between, no longer
+// finds part of it in that cache (B2 H8 KV 32768, 256 MiB, the same call back to
+// back 43.7 -> 45.9 us; on rotating sets 53.7 -> 46.7). A decode loop reads the
+// other layers' K/V between two steps of one layer, so the second is its case.
 constexpr int64_t kNonTemporalBytes = int64_t(128) << 20;
 __device__ __forceinline__ bool non_temporal_kv(const FwdParams& p, int len, int64_t row_bytes) {
   return p.q_tiles == 1 && p.dim % 64 == 0 &&
