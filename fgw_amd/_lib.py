@@ -59,6 +59,21 @@ class Schedule(ctypes.Structure):
                 ("block_keys", c_int32)]
 
 
+# Kernel names by id, and what a call launches (fgw_amd/csrc/fmha_launch_info.h: a
+# diagnostic of this library, not part of the C ABI).
+KERNELS = ("query", "query_groups", "query_eight_waves", "key", "key_groups", "decode",
+           "prefill", "prefill_groups", "prefill_padded", "half_tiles", "half_tiles_padded")
+
+
+class LaunchInfo(ctypes.Structure):
+    _fields_ = [("kernel", c_int32), ("threads", c_int32), ("rows_per_item", c_int32),
+                ("q_tiles", c_int32), ("work_items", c_int32), ("grid", c_int32)]
+
+    @property
+    def name(self) -> str:
+        return KERNELS[self.kernel]
+
+
 # name -> (argtypes); every function returns int.
 SIGNATURES = {
     "fgw_mha_abi_version": (),
@@ -102,6 +117,9 @@ def load() -> ctypes.CDLL:
             fn = getattr(lib, name)
             fn.argtypes = list(argtypes)
             fn.restype = ctypes.c_char_p if name == "fgw_mha_last_error" else ctypes.c_int
+        lib.fgw_internal_launch_info.argtypes = [ctypes.POINTER(Shape), ctypes.POINTER(Plan),
+                                                 ctypes.POINTER(LaunchInfo)]
+        lib.fgw_internal_launch_info.restype = ctypes.c_int
         version = lib.fgw_mha_abi_version()
         if version != ABI_VERSION:
             raise RuntimeError(f"{LIBRARY} has ABI {version}, expected {ABI_VERSION}; rebuild it")
@@ -144,4 +162,11 @@ def plan(shape: Shape, request: Request, device: DeviceInfo) -> Plan:
     out = Plan()
     check(load().fgw_mha_plan(ctypes.byref(shape), ctypes.byref(request), ctypes.byref(device),
                               ctypes.byref(out)))
+    return out
+
+
+def launch_info(shape: Shape, plan: Plan) -> LaunchInfo:
+    """The kernel variant, items and programs that a call of this plan launches."""
+    out = LaunchInfo()
+    check(load().fgw_internal_launch_info(ctypes.byref(shape), ctypes.byref(plan), ctypes.byref(out)))
     return out

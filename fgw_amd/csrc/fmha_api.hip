@@ -13,6 +13,7 @@
 #include "fmha_decode.h"
 #include "fmha_half.h"
 #include "fmha_kernel.h"
+#include "fmha_launch_info.h"
 #include "fmha_prefill.h"
 #include "fmha_registry.h"
 
@@ -534,43 +535,6 @@ bool dual_takes(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
          capacity - hidden >= kDualMinKeys * (p->num_splits > 1 ? p->num_splits : 1);
 }
 
-// The kernel of a plan: the layout's own (`fallback`) or one of its variants.
-// - Key layout, Sq = 1: the single-token kernel where decode_takes it.
-// - Key and query layouts: the row-group kernel where the whole-block fast path
-//   would not hold (pages that a block, 32 keys in the key layout and 64 in the
-//   query layout, straddles, or a head dim below its tile) and an instruction's
-//   rows (512 / tile of them) lie in one page, and in the key layout where K/V
-//   may be large enough for its non-temporal loads (non_temporal_kv looks
-//   at the lengths). Measured against the plain kernel: B4 H16 Q8 KV <= 8192
-//   causal 44.1 -> 42.5 us, with pages of 16 66.7 -> 42.2; B8 H32 Q4 KV <= 2048
-//   pages of 16 65.9 -> 39.0; B2 H8 Q16 KV 32768 54.6 -> 48.9; B16 H8 Q20 D96
-//   pages of 48 21.4 -> 15.7; B8 H32 Q5 D32 pages of 16 71.5 -> 38.6. Small
-//   calls of whole blocks keep the plain kernel (B1 H8 Q4 D64 KV 512 9.35
-//   against 9.57, B2 H8 Q16 KV 2048 13.4 against 13.6).
-// - Query layout: the eight-wave kernel where dual_takes it.
-// - Prefill layout: a row-group variant where the whole-block fast path would
-//   not hold (pages that a 64-key block straddles, or a head dim below its
-//   tile) and an instruction's rows (512 / tile of them) still lie in one page.
-FwdLaunchFn kernel_of(const fgw_mha_shape* s, const fgw_mha_plan_t* p, FwdLaunchFn fallback) {
-  const bool bf16 = s->dtype == FGW_MHA_BFLOAT16;
-  FwdLaunchFn f = nullptr;
-  if (p->layout == kLayoutKey && s->sq == 1 &&
-      decode_takes(p->dim_padded, (int64_t)s->heads * s->dim * 2, s->page_size))
-    f = decode_entry(bf16, p->dim_padded);
-  else if (p->layout != kLayoutPrefill && s->page_size % (512 / p->dim_padded) == 0 &&
-           (s->page_size % (p->layout == kLayoutKey ? 32 : 64) || s->dim != p->dim_padded ||
-            (p->layout == kLayoutKey && 4 * (int64_t)s->batch * s->width * s->page_size * s->heads *
-                                            s->dim >= kNonTemporalBytes)))
-    f = groups_entry(bf16, p->dim_padded, p->layout,
-                     p->stages == default_stages(p->layout, p->dim_padded) ? 0 : p->stages);
-  else if (dual_takes(s, p))
-    f = dual_entry(bf16);
-  else if (p->layout == kLayoutPrefill && (s->page_size % 64 || s->dim != p->dim_padded) &&
-           s->page_size % (512 / p->dim_padded) == 0)
-    f = prefill_rows_entry(bf16, p->dim_padded, s->dim == p->dim_padded ? kRowsGroup : kRowsPadded);
-  return f ? f : fallback;
-}
-
 constexpr int kRowsHalfTile = HCfg<true, 128, kRowsGroup>::ROWS_TILE;
 
 // Key blocks on the critical path of a direct plan with query tiles of `rows`
@@ -618,30 +582,91 @@ bool half_tiles(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
          0.95 * critical_steps(s, 2 * kRowsHalfTile, 1, 1.0);
 }
 
+// The kernel of a plan: the layout's own or one of its variants.
+// - Key layout, Sq = 1: the single-token kernel where decode_takes it.
+// - Key and query layouts: the row-group kernel where the whole-block fast path
+//   would not hold (pages that a block, 32 keys in the key layout and 64 in the
+//   query layout, straddles, or a head dim below its tile) and an instruction's
+//   rows (512 / tile of them) lie in one page, and in the key layout where K/V
+//   may be large enough for its non-temporal loads (non_temporal_kv looks
+//   at the lengths). Measured against the plain kernel: B4 H16 Q8 KV <= 8192
+//   causal 44.1 -> 42.5 us, with pages of 16 66.7 -> 42.2; B8 H32 Q4 KV <= 2048
+//   pages of 16 65.9 -> 39.0; B2 H8 Q16 KV 32768 54.6 -> 48.9; B16 H8 Q20 D96
+//   pages of 48 21.4 -> 15.7; B8 H32 Q5 D32 pages of 16 71.5 -> 38.6. Small
+//   calls of whole blocks keep the plain kernel (B1 H8 Q4 D64 KV 512 9.35
+//   against 9.57, B2 H8 Q16 KV 2048 13.4 against 13.6).
+// - Query layout: the eight-wave kernel where dual_takes it.
+// - Prefill layout: a row-group variant where the whole-block fast path would
+//   not hold (pages that a 64-key block straddles, or a head dim below its
+//   tile) and an instruction's rows (512 / tile of them) still lie in one page;
+//   the half-tile kernel where half_tiles takes the plan.
+Kernel kernel_of(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
+  const bool row_groups = s->page_size % (512 / p->dim_padded) == 0;
+  const bool padded = s->dim != p->dim_padded;
+  if (p->layout == kLayoutPrefill) {
+    if (half_tiles(s, p)) return padded ? kKernelHalfPadded : kKernelHalf;
+    if (!row_groups || !(s->page_size % 64 || padded)) return kKernelPrefill;
+    return padded ? kKernelPrefillPadded : kKernelPrefillGroups;
+  }
+  const bool key = p->layout == kLayoutKey;
+  if (key && s->sq == 1 &&
+      decode_takes(p->dim_padded, (int64_t)s->heads * s->dim * 2, s->page_size))
+    return kKernelDecode;
+  if (row_groups && (s->page_size % (key ? 32 : 64) || padded ||
+                     (key && 4 * (int64_t)s->batch * s->width * s->page_size * s->heads * s->dim >=
+                                 kNonTemporalBytes)))
+    return key ? kKernelKeyGroups : kKernelQueryGroups;
+  if (dual_takes(s, p)) return kKernelQueryDual;
+  return key ? kKernelKey : kKernelQuery;
+}
+
+FwdLaunchFn launch_fn(const fgw_mha_shape* s, const fgw_mha_plan_t* p, Kernel kernel) {
+  const bool bf16 = s->dtype == FGW_MHA_BFLOAT16;
+  const int dpad = p->dim_padded;
+  const int stages = p->stages == default_stages(p->layout, dpad) ? 0 : p->stages;
+  switch (kernel) {
+    case kKernelQueryGroups:
+    case kKernelKeyGroups: return groups_entry(bf16, dpad, p->layout, stages);
+    case kKernelQueryDual: return dual_entry(bf16);
+    case kKernelDecode: return decode_entry(bf16, dpad);
+    case kKernelPrefillGroups: return prefill_rows_entry(bf16, dpad, kRowsGroup);
+    case kKernelPrefillPadded: return prefill_rows_entry(bf16, dpad, kRowsPadded);
+    case kKernelHalf: return half_entry(bf16, dpad, kRowsGroup);
+    case kKernelHalfPadded: return half_entry(bf16, dpad, kRowsPadded);
+    default: return fwd_entry(bf16, dpad, p->layout, stages).launch;
+  }
+}
+
+// What a call of this plan launches. The half-tile kernel's items are half the
+// plan's query tiles, so that it has its own count of them; a plan with fewer
+// programs than items keeps its grid.
+LaunchInfo launch_info(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
+  LaunchInfo i;
+  i.kernel = kernel_of(s, p);
+  const bool half = i.kernel == kKernelHalf || i.kernel == kKernelHalfPadded;
+  i.threads = p->layout == kLayoutPrefill || i.kernel == kKernelDecode || i.kernel == kKernelQueryDual
+                  ? 512 : 256;
+  i.rows_per_item = i.kernel == kKernelDecode ? 1 : (half ? kRowsHalfTile : p->rows_per_tile);
+  i.q_tiles = half ? (s->sq + kRowsHalfTile - 1) / kRowsHalfTile : p->q_tiles;
+  i.work_items = half ? s->batch * s->heads * i.q_tiles : p->work_items;
+  i.grid = p->grid == p->work_items || p->grid > i.work_items ? i.work_items : p->grid;
+  return i;
+}
+
 // `whole`: the partial kernel of a full call, whose merge follows (a
 // tile-balanced plan's one-split tiles then write their output directly).
 int launch_partial_kernel(const fgw_mha_shape* s, const fgw_mha_plan_t* p,
                           const fgw_mha_tensors* t, int mode, hipStream_t stream,
                           bool whole = false, int32_t* arrivals = nullptr) {
-  const int stages = p->stages == default_stages(p->layout, p->dim_padded) ? 0 : p->stages;
-  const FwdEntry e = fwd_entry(s->dtype == FGW_MHA_BFLOAT16, p->dim_padded, p->layout, stages);
-  if (!e.launch) return fail(FGW_MHA_EUNSUPPORTED, "no kernel for dim tile %d", p->dim_padded);
+  const LaunchInfo info = launch_info(s, p);
+  const FwdLaunchFn launch = launch_fn(s, p, (Kernel)info.kernel);
+  if (!launch) return fail(FGW_MHA_EUNSUPPORTED, "no kernel for dim tile %d", p->dim_padded);
   FwdParams f = make_params(s, p, t, mode);
+  f.q_tiles = info.q_tiles;
+  f.work = info.work_items;
   f.split_direct = whole && mode == 1 && tile_balanced(p->layout, s->causal, p->split_keys);
   f.arrivals = mode == 1 ? arrivals : nullptr;
-  const FwdLaunchFn launch = kernel_of(s, p, e.launch);
-  if (half_tiles(s, p)) {
-    // Twice the items; a plan with fewer programs than items keeps its grid.
-    f.q_tiles = (s->sq + kRowsHalfTile - 1) / kRowsHalfTile;
-    f.work = s->batch * s->heads * f.q_tiles;
-    const int grid = p->grid == p->work_items ? f.work : (p->grid < f.work ? p->grid : f.work);
-    const FwdLaunchFn half =
-        half_entry(s->dtype == FGW_MHA_BFLOAT16, p->dim_padded,
-                   s->dim == p->dim_padded ? kRowsGroup : kRowsPadded);
-    const hipError_t err = half(f, grid, stream);
-    return err == hipSuccess ? FGW_MHA_OK : hip_fail(err, "forward kernel launch");
-  }
-  const hipError_t err = launch(f, p->grid, stream);
+  const hipError_t err = launch(f, info.grid, stream);
   return err == hipSuccess ? FGW_MHA_OK : hip_fail(err, "forward kernel launch");
 }
 
@@ -844,6 +869,14 @@ int fgw_mha_plan(const fgw_mha_shape* s, const fgw_mha_request* req,
   out->stages = stages;
   out->arrival_counters = (int32_t)fused_merge_counters(s, layout, splits, rows, tasks);
   return FGW_MHA_OK;
+}
+
+int fgw_internal_launch_info(const fgw_mha_shape* s, const fgw_mha_plan_t* p, LaunchInfo* info) {
+  int rc = check_shape(s);
+  if (!rc) rc = check_plan(s, p);
+  if (!rc && !info) rc = fail(FGW_MHA_EINVAL, "info is NULL");
+  if (!rc) *info = launch_info(s, p);
+  return rc;
 }
 
 int fgw_mha_fwd(const fgw_mha_shape* s, const fgw_mha_plan_t* p, const fgw_mha_tensors* t,

@@ -145,6 +145,12 @@ class _Launch(_launch.Launcher):
             self.merge_kernel = self._merge
 
     # -- helpers -----------------------------------------------------------
+    @property
+    def launch_info(self) -> _lib.LaunchInfo:
+        """The kernel variant that a call launches, its items and programs (a
+        diagnostic: the planned attributes above describe the layout's tiling)."""
+        return _lib.launch_info(self._shape, self._plan)
+
     def _check(self, q, k, v, table, lengths):
         """Checks of the component calls (partial); the full call makes the
         same checks in C++."""

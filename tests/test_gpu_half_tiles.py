@@ -26,6 +26,7 @@ def _check(b, sq, h, d, page, lengths, dtype, causal, **plan):
     kern = build_kernel(b, sq, h, d, k.shape[0], width, page, causal,
                         "float16" if dtype == torch.float16 else "bfloat16", 0, layout="prefill",
                         num_splits=1, **plan)
+    assert kern.launch_info.name == ("half_tiles" if d in (64, 128) else "half_tiles_padded")
     got = kern(*[x.cuda() for x in (q, k, v, table, lengths)]).cpu()
     rtol, atol = O.TOLERANCES[dtype]
     torch.testing.assert_close(got, O.chunked_reference(q, k, v, table, lengths, page, causal),

@@ -1,5 +1,5 @@
 """The prefill layout's per-instruction variants against the oracle: pages that a
-64-key block straddles and head dims 80 and 96.
+64-key block straddles and head dims below their tile.
 
 Where they can go wrong: caches that end inside an instruction's rows, page
 sizes of one instruction's rows and off the powers of two, page ids outside
@@ -17,7 +17,11 @@ from oracle import mha_oracle as O
 gpu = pytest.mark.gpu
 
 
-def _check(b, sq, h, d, page, lengths, dtype, causal, outside=False, **plan):
+def _rows_kernel(d):
+    return "prefill_groups" if d in (64, 128) else "prefill_padded"
+
+
+def _check(b, sq, h, d, page, lengths, dtype, causal, outside=False, kernel=None, **plan):
     from fgw_amd.operators.mha.current import build_kernel
     width = -(-max(lengths) // page)
     q, k, v, table = O.make_inputs(("rows", b, sq, h, d, page, width), 5, dtype)
@@ -34,6 +38,8 @@ def _check(b, sq, h, d, page, lengths, dtype, causal, outside=False, **plan):
     kern = build_kernel(b, sq, h, d, k.shape[0], width, page, causal,
                         "float16" if dtype == torch.float16 else "bfloat16", 0, layout="prefill",
                         **plan)
+    if kernel:
+        assert kern.launch_info.name == kernel
     got = kern(*[x.cuda() for x in (q, k, v, table, lengths)]).cpu()
     rtol, atol = O.TOLERANCES[dtype]
     torch.testing.assert_close(got, O.chunked_reference(q, ek, ev, etable, lengths, page, causal),
@@ -49,29 +55,43 @@ def _check(b, sq, h, d, page, lengths, dtype, causal, outside=False, **plan):
     (128, 6, torch.bfloat16), (96, 5, torch.float16), (112, 16, torch.bfloat16)])
 def test_ragged_pages_match_the_oracle(d, page, dtype, causal):
     lengths = [0, 1, 3, 63, 64, 65, 130, 257, 300]
-    for splits in (1, 2):
-        _check(len(lengths), 257, 2, d, page, lengths, dtype, causal, num_splits=splits)
+    general = (d, page) in ((128, 6), (96, 5))  # pages that split a load instruction's rows
+    for splits in (1, 2):  # (unsplit, some of these run on the half-tile kernel)
+        _check(len(lengths), 257, 2, d, page, lengths, dtype, causal, num_splits=splits,
+               kernel=None if splits == 1 else "prefill" if general else _rows_kernel(d))
 
 
 @gpu
 @pytest.mark.parametrize("d,page", [(128, 16), (64, 16), (96, 32)])
 def test_more_blocks_than_a_window(d, page):
-    _check(1, 300, 1, d, page, [4500], torch.bfloat16, False, num_splits=1)
-    _check(2, 260, 1, d, page, [4500, 2111], torch.bfloat16, True, num_splits=2)
+    keys = 8704 if d == 64 else 4500  # 68 blocks per split, 35 and 36
+    _check(1, 300, 1, d, page, [keys], torch.bfloat16, False, num_splits=2, kernel=_rows_kernel(d))
+    _check(2, 260, 1, d, page, [keys, 2111], torch.bfloat16, True, num_splits=2,
+           kernel=_rows_kernel(d))
 
 
 @gpu
-@pytest.mark.parametrize("d,page", [(96, 64), (128, 16), (80, 16)])
+@pytest.mark.parametrize("d,page", [(96, 64), (128, 16), (80, 16), (128, 48)])
 def test_several_items_per_program(d, page):
+    """At most 320 keys: an unsplit item is too short for the half-tile kernel."""
     for grid in (3, 8):
-        _check(2, 600, 3, d, page, [200, 333], torch.float16, False, num_splits=1,
-               persistent_programs=grid)
+        for causal in (False, True):
+            _check(2, 600, 3, d, page, [200, 288], torch.float16, causal, num_splits=1,
+                   persistent_programs=grid, kernel=_rows_kernel(d))
+
+
+@gpu
+def test_several_items_per_program_head_dim_64():
+    """531 query tiles: more than the half-tile kernel takes."""
+    _check(1, 15000, 9, 64, 16, [250], torch.bfloat16, False, num_splits=1, persistent_programs=48,
+           kernel="prefill_groups")
 
 
 @gpu
 @pytest.mark.parametrize("d,page", [(128, 16), (96, 64)])
 def test_page_ids_outside_the_pool_read_as_zeros(d, page):
-    _check(2, 200, 2, d, page, [320, 177], torch.bfloat16, False, outside=True, num_splits=1)
+    _check(2, 200, 2, d, page, [320, 177], torch.bfloat16, False, outside=True, num_splits=1,
+           kernel=_rows_kernel(d))
 
 
 @gpu
@@ -90,7 +110,7 @@ def test_more_causal_items_than_cus(sq, lengths, plan):
     lengths = torch.tensor(lengths, dtype=torch.int32)
     kern = build_kernel(b, sq, h, d, k.shape[0], width, page, True, "float16", 0, layout="prefill",
                         **plan)
-    assert kern.compute_work > 256
+    assert kern.compute_work > 256 and kern.launch_info.name == "prefill"
     got = kern(*[x.cuda() for x in (q, k, v, table, lengths)]).cpu()
     rtol, atol = O.TOLERANCES[torch.float16]
     torch.testing.assert_close(got, O.chunked_reference(q, k, v, table, lengths, page, True),

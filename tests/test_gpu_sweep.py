@@ -5,8 +5,9 @@ length, ragged lengths, causal, dtype, split request and layout from a fixed
 seed, poisons every unread pool row with NaN and checks the output against
 the oracle at the reference tolerances, with exactly-zero rows where no key
 is visible. Key-layout plans at head-dim tile 128 also run on the
-single-stage key kernel, which must give the same bits. The draws stay small
-enough for the oracle to finish in seconds.
+single-stage key kernel, which must give the same bits (the single-token
+kernel has no stages: Sq = 1 is compared at pages that it does not take).
+The draws stay small enough for the oracle to finish in seconds.
 """
 import random
 
@@ -55,7 +56,7 @@ def test_random_case(i):
                         num_splits=splits, layout=layout, cache_lengths=tuple(lengths))
     dev = [x.cuda() for x in (q, k, v, table, lt)]
     got = kern(*dev)
-    if kern.layout == "key" and kern.dim_padded == 128:
+    if kern.layout == "key" and kern.dim_padded == 128 and kern.launch_info.name != "decode":
         # The single-stage key kernel computes the same bits.
         single = build_kernel(b, sq, h, d, k.shape[0], width, page, causal,
                               "float16" if dtype == torch.float16 else "bfloat16", 0,
@@ -113,7 +114,7 @@ def test_random_balanced_case(i):
     got = kern(*dev)
     parts, lse = kern.partial_kernel(*dev)
     merged = kern.merge_kernel(parts, lse, dev[4])
-    if kern.dim_padded == 128:
+    if kern.dim_padded == 128 and kern.launch_info.name != "decode":
         single = build_kernel(b, sq, h, d, k.shape[0], width, page, causal,
                               "float16" if dtype == torch.float16 else "bfloat16", 0,
                               num_splits=splits, layout="key", split_keys=split_keys, stages=1)
@@ -129,3 +130,26 @@ def test_random_balanced_case(i):
     if causal:
         visible = (visible - sq + torch.arange(sq)[None, :] + 1).clamp_min(0)
     assert torch.count_nonzero(got[visible == 0]).item() == 0, label
+
+
+@pytest.mark.parametrize("split_keys", [None, 150])
+@pytest.mark.parametrize("d,page", [(128, 6), (112, 10)])
+def test_single_token_stages_agree(d, page, split_keys):
+    """Pages that split a load instruction's rows keep the MFMA key kernel at Sq = 1, whose
+    single- and double-stage instantiations compute the same bits."""
+    from fgw_amd.operators.mha.current import build_kernel
+    b, h, width = 3, 4, 1200 // page
+    q, k, v, table = O.make_inputs(("stages", b, 1, h, d, page, width), 3, torch.bfloat16)
+    lt = torch.tensor([width * page, 0, 517], dtype=torch.int32)
+    k, v = O.poison_unread(k, v, table, lt, page)
+    dev = [x.cuda() for x in (q, k, v, table, lt)]
+    outs = []
+    for stages in (1, 2):
+        kern = build_kernel(b, 1, h, d, k.shape[0], width, page, False, "bfloat16", 0, num_splits=8,
+                            layout="key", split_keys=split_keys, stages=stages)
+        assert kern.launch_info.name == "key" and kern.stages == stages
+        outs.append(kern(*dev))
+    assert torch.equal(*outs)
+    rtol, atol = O.TOLERANCES[torch.bfloat16]
+    torch.testing.assert_close(outs[0].cpu(), O.reference(q, k, v, table, lt, page, False),
+                               rtol=rtol, atol=atol)
