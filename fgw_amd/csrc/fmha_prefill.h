@@ -402,12 +402,8 @@ __device__ __forceinline__ void mask_from(f32x16 (&s)[C::ST], int lim) {
     }
 }
 
-// Aligned to a page: the kernel is about 110 KB of unrolled code, more than the
-// instruction cache, and its speed moved by up to 1% with its place in the
-// code object (Q4096 0.994-1.01x, Q32768 0.985-1.002x over builds that differ
-// in other kernels only; page-aligned 1.009x on both).
 template <class C>
-__global__ __attribute__((aligned(4096))) __launch_bounds__(C::THREADS) void prefill_kernel(FwdParams p_arg,
+__global__ __launch_bounds__(C::THREADS) void prefill_kernel(FwdParams p_arg,
                                                              const int32_t* __restrict__ table,
                                                              const int32_t* __restrict__ lengths) {
   __shared__ __attribute__((aligned(1024))) unsigned char smem[C::LDS_BYTES];
