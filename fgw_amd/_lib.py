@@ -61,13 +61,15 @@ class Schedule(ctypes.Structure):
 
 # Kernel names by id, and what a call launches (fgw_amd/csrc/fmha_launch_info.h: a
 # diagnostic of this library, not part of the C ABI).
-KERNELS = ("query", "query_groups", "query_eight_waves", "key", "key_groups", "decode",
-           "prefill", "prefill_groups", "prefill_padded", "half_tiles", "half_tiles_padded")
+KERNELS = ("query", "query_groups", "query_eight_waves", "key", "key_groups", "key_stream",
+           "decode", "prefill", "prefill_groups", "prefill_padded", "half_tiles",
+           "half_tiles_padded")
 
 
 class LaunchInfo(ctypes.Structure):
     _fields_ = [("kernel", c_int32), ("threads", c_int32), ("rows_per_item", c_int32),
-                ("q_tiles", c_int32), ("work_items", c_int32), ("grid", c_int32)]
+                ("q_tiles", c_int32), ("work_items", c_int32), ("grid", c_int32),
+                ("stream_bytes", c_int64)]
 
     @property
     def name(self) -> str:

@@ -36,6 +36,8 @@ FGW_MHA_FOR_PREFILL_ROWS(FGW_MHA_EXTERN_HALF, true)
 FGW_MHA_FOR_PREFILL_ROWS(FGW_MHA_EXTERN_HALF, false)
 FGW_MHA_FOR_GROUPS(FGW_MHA_EXTERN_GROUPS, true)
 FGW_MHA_FOR_GROUPS(FGW_MHA_EXTERN_GROUPS, false)
+FGW_MHA_FOR_STREAM(FGW_MHA_EXTERN_STREAM, true)
+FGW_MHA_FOR_STREAM(FGW_MHA_EXTERN_STREAM, false)
 extern FGW_MHA_INSTANTIATE_DUAL(true)
 extern FGW_MHA_INSTANTIATE_DUAL(false)
 FGW_MHA_FOR_DECODE(FGW_MHA_EXTERN_DECODE, true)
@@ -78,6 +80,15 @@ FwdLaunchFn groups_entry(bool bf16, int dpad, int layout, int stages) {
     return &launch_fwd<BF, DP, LY, ST, kGroups>;
   FGW_MHA_FOR_GROUPS(FGW_GROUPS_ENTRY, true)
   FGW_MHA_FOR_GROUPS(FGW_GROUPS_ENTRY, false)
+  return nullptr;
+}
+
+FwdLaunchFn stream_entry(bool bf16, int dpad, int stages) {
+#define FGW_STREAM_ENTRY(BF, DP, ST)                 \
+  if (bf16 == BF && dpad == DP && stages == ST)      \
+    return &launch_fwd<BF, DP, kLayoutKey, ST, kStream>;
+  FGW_MHA_FOR_STREAM(FGW_STREAM_ENTRY, true)
+  FGW_MHA_FOR_STREAM(FGW_STREAM_ENTRY, false)
   return nullptr;
 }
 
@@ -489,6 +500,7 @@ FwdParams make_params(const fgw_mha_shape* s, const fgw_mha_plan_t* p, const fgw
   f.mode = mode;
   f.split_keys = mode == 1 ? p->split_keys : 0;
   f.split_direct = 0;
+  f.stream_bytes = 0;
   page_divisor((uint32_t)s->page_size, &f.page_magic, &f.page_shift);
   f.scale_log2 = (float)(1.4426950408889634 / __builtin_sqrt((double)s->dim));
   f.segs = nullptr;
@@ -583,23 +595,43 @@ bool half_tiles(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
 }
 
 // The kernel of a plan: the layout's own or one of its variants.
-// - Key layout, Sq = 1: the single-token kernel where decode_takes it.
+// - Key layout, Sq = 1: the single-token kernel where decode_takes it, but for
+//   whole blocks of large K/V at tiles 64 and 128, where the key kernel's DMA
+//   keeps more bytes in flight than the single-token kernel's registers. At 128
+//   the line is 128 MiB: repeated, rotating and shared pages, as ratios to the key
+//   kernel, 0.98 / 0.98 / 1.01 there, 1.00 / 1.00 / 1.05 at 192 MiB, 1.03 / 1.01 /
+//   1.14 from 256 MiB; 0.88-1.01 below. At 64 it is the last-level cache's size
+//   (the key kernel gains more from non-temporal loads): 0.97-1.02 and 0.65-0.99
+//   with shared pages below, 1.00-1.24 from there on. Tiles 32 (0.6-0.97) and 256
+//   (0.72-1.06) have no such line.
+// - Key layout: the kernel with non-temporal loads where the table can hold more K/V
+//   than the last-level cache.
 // - Key and query layouts: the row-group kernel where the whole-block fast path
 //   would not hold (pages that a block, 32 keys in the key layout and 64 in the
 //   query layout, straddles, or a head dim below its tile) and an instruction's
-//   rows (512 / tile of them) lie in one page, and in the key layout where K/V
-//   may be large enough for its non-temporal loads (non_temporal_kv looks
-//   at the lengths). Measured against the plain kernel: B4 H16 Q8 KV <= 8192
-//   causal 44.1 -> 42.5 us, with pages of 16 66.7 -> 42.2; B8 H32 Q4 KV <= 2048
-//   pages of 16 65.9 -> 39.0; B2 H8 Q16 KV 32768 54.6 -> 48.9; B16 H8 Q20 D96
-//   pages of 48 21.4 -> 15.7; B8 H32 Q5 D32 pages of 16 71.5 -> 38.6. Small
-//   calls of whole blocks keep the plain kernel (B1 H8 Q4 D64 KV 512 9.35
-//   against 9.57, B2 H8 Q16 KV 2048 13.4 against 13.6).
+//   rows (512 / tile of them) lie in one page. Measured against the plain kernel:
+//   B4 H16 Q8 KV <= 8192 causal pages of 16 66.7 -> 42.2 us; B8 H32 Q4 KV <= 2048
+//   pages of 16 65.9 -> 39.0; B16 H8 Q20 D96 pages of 48 21.4 -> 15.7; B8 H32 Q5
+//   D32 pages of 16 71.5 -> 38.6. With whole blocks it is the slower one (B64 H8
+//   Sq 8 KV 4096, shared pages, cached loads: 82 us against 72).
 // - Query layout: the eight-wave kernel where dual_takes it.
 // - Prefill layout: a row-group variant where the whole-block fast path would
 //   not hold (pages that a 64-key block straddles, or a head dim below its
 //   tile) and an instruction's rows (512 / tile of them) still lie in one page;
 //   the half-tile kernel where half_tiles takes the plan.
+constexpr int64_t kCacheBytes = int64_t(256) << 20;      // last-level cache
+constexpr int64_t kDecodeMaxBytes = int64_t(128) << 20;  // decode_kernel at tile 128, whole blocks
+
+// K and V bytes that the call's items read at full table capacity, and of the
+// rows they lie in (requests may share pages: not more than the pool's).
+int64_t capacity_bytes(const fgw_mha_shape* s) {
+  return 4 * (int64_t)s->batch * s->width * s->page_size * s->heads * s->dim;
+}
+int64_t max_kv_bytes(const fgw_mha_shape* s) {
+  const int64_t pool = 4 * s->pool_rows * s->heads * s->dim;
+  return pool < capacity_bytes(s) ? pool : capacity_bytes(s);
+}
+
 Kernel kernel_of(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
   const bool row_groups = s->page_size % (512 / p->dim_padded) == 0;
   const bool padded = s->dim != p->dim_padded;
@@ -609,15 +641,44 @@ Kernel kernel_of(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
     return padded ? kKernelPrefillPadded : kKernelPrefillGroups;
   }
   const bool key = p->layout == kLayoutKey;
+  const bool whole = s->page_size % (key ? 32 : 64) == 0 && !padded;  // whole blocks
+  const int64_t bytes = capacity_bytes(s);
   if (key && s->sq == 1 &&
-      decode_takes(p->dim_padded, (int64_t)s->heads * s->dim * 2, s->page_size))
+      decode_takes(p->dim_padded, (int64_t)s->heads * s->dim * 2, s->page_size) &&
+      !(whole && ((p->dim_padded == 128 && bytes >= kDecodeMaxBytes) ||
+                  (p->dim_padded == 64 && bytes >= kCacheBytes))))
     return kKernelDecode;
-  if (row_groups && (s->page_size % (key ? 32 : 64) || padded ||
-                     (key && 4 * (int64_t)s->batch * s->width * s->page_size * s->heads * s->dim >=
-                                 kNonTemporalBytes)))
-    return key ? kKernelKeyGroups : kKernelQueryGroups;
+  if (row_groups && !whole) return key ? kKernelKeyGroups : kKernelQueryGroups;
+  if (key && p->q_tiles == 1 && p->dim_padded >= 64 && max_kv_bytes(s) > kCacheBytes)
+    return kKernelKeyStream;
   if (dual_takes(s, p)) return kKernelQueryDual;
   return key ? kKernelKey : kKernelQuery;
+}
+
+// FwdParams::stream_bytes of a plan's kernel (0: it has no non-temporal loads, or
+// its K/V cannot reach the limit). Non-temporal loads pay where nothing else of
+// the call reads the rows again: one query tile, head rows that fill whole
+// 128-byte lines (heads would share them; D 48 measured 1.11x slower), no shared
+// pages (stream_kv).
+// - Whole blocks: above the last-level cache. A call that is repeated on a set of
+//   up to that size finds it there, and the loads past it made that slower
+//   (repeated on one set / over three rotating ones, as ratios to cached loads:
+//   BF16 D128 Sq 8 KV 8192, 256 MiB 1.07 / 0.91; Sq 1 192 MiB 1.06 / 0.91; 320 MiB
+//   0.95 / 0.91; 512 MiB 0.88 / 0.90; D64 256 MiB 1.07 / 0.83, 320 MiB 0.83 / 0.81).
+// - Small pages and padded head dims, and D 256 at Sq 1: from half of it on. Their
+//   kernels are that much faster than the ones they replace that both kinds of
+//   caller gain (B8 H8 KV 8192 pages of 16, 256 MiB: repeated 60.8 -> 46.2 us,
+//   rotating 70.4 -> 48.3; with cached loads 45.0 and 54.6).
+int64_t stream_bytes_of(const fgw_mha_shape* s, const fgw_mha_plan_t* p, Kernel kernel) {
+  if (p->q_tiles > 1 || s->dim % 64 ||
+      !(kernel == kKernelKeyStream || kernel == kKernelDecode || kernel == kKernelKeyGroups ||
+        kernel == kKernelQueryGroups))
+    return 0;
+  const bool whole = s->page_size % 32 == 0 && s->dim == p->dim_padded;
+  const bool cache = kernel == kKernelKeyStream ||
+                     (kernel == kKernelDecode && whole && p->dim_padded < 256);
+  const int64_t limit = cache ? kCacheBytes : kCacheBytes / 2;
+  return max_kv_bytes(s) > limit ? limit : 0;
 }
 
 FwdLaunchFn launch_fn(const fgw_mha_shape* s, const fgw_mha_plan_t* p, Kernel kernel) {
@@ -627,6 +688,7 @@ FwdLaunchFn launch_fn(const fgw_mha_shape* s, const fgw_mha_plan_t* p, Kernel ke
   switch (kernel) {
     case kKernelQueryGroups:
     case kKernelKeyGroups: return groups_entry(bf16, dpad, p->layout, stages);
+    case kKernelKeyStream: return stream_entry(bf16, dpad, stages);
     case kKernelQueryDual: return dual_entry(bf16);
     case kKernelDecode: return decode_entry(bf16, dpad);
     case kKernelPrefillGroups: return prefill_rows_entry(bf16, dpad, kRowsGroup);
@@ -643,6 +705,7 @@ FwdLaunchFn launch_fn(const fgw_mha_shape* s, const fgw_mha_plan_t* p, Kernel ke
 LaunchInfo launch_info(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
   LaunchInfo i;
   i.kernel = kernel_of(s, p);
+  i.stream_bytes = stream_bytes_of(s, p, (Kernel)i.kernel);
   const bool half = i.kernel == kKernelHalf || i.kernel == kKernelHalfPadded;
   i.threads = p->layout == kLayoutPrefill || i.kernel == kKernelDecode || i.kernel == kKernelQueryDual
                   ? 512 : 256;
@@ -662,6 +725,7 @@ int launch_partial_kernel(const fgw_mha_shape* s, const fgw_mha_plan_t* p,
   const FwdLaunchFn launch = launch_fn(s, p, (Kernel)info.kernel);
   if (!launch) return fail(FGW_MHA_EUNSUPPORTED, "no kernel for dim tile %d", p->dim_padded);
   FwdParams f = make_params(s, p, t, mode);
+  f.stream_bytes = info.stream_bytes;
   f.q_tiles = info.q_tiles;
   f.work = info.work_items;
   f.split_direct = whole && mode == 1 && tile_balanced(p->layout, s->causal, p->split_keys);

@@ -20,16 +20,17 @@
 // known and its V registers as soon as its products are done, so that one of
 // the two is always in flight.
 //
-// What bounds it: HBM reads for long caches (8 waves keep 64 KB in flight per
-// workgroup), the chain length -> table -> K -> V -> combine for short ones.
-// Measured against the MFMA key kernel at Sq = 1 (D 128 unless said, K/V from
-// three rotating sets): B16 H16 KV 1024-4096 pages of 16 125 -> 59-68 us, B8
-// H32 KV 4096 98.5 -> 89.9 us (6.0 TB/s), B2 H8 KV 32768 53.5 -> 46.6 us, B8
-// H32 KV 2048 D 96 65 -> 33 us, D 64 KV 4096 pages of 16 96 -> 53 us, B1 H1
-// KV 512 8.2 -> 7.8 us. Steps of 32 keys at D 128 (twice the registers, one
-// workgroup per CU) measured 0-8% slower except on the shortest calls (B1 H1
-// KV 512 7.4 us); 4 waves 1-7% slower; the heads of a key range as neighbours
-// instead of a head's splits 7% slower at B2 H8 KV 32768.
+// What bounds it: memory reads for long caches (8 waves keep 64 KB in flight per
+// workgroup; reads that the caches serve are bound by that and by the vector ALU, where
+// the MFMA key kernel's DMA keeps 128 KB in flight: kernel_of in fmha_api.hip draws
+// the line), the chain length -> table -> K -> V -> combine for short ones.
+// Measured against the MFMA key kernel at Sq = 1 (D 128 unless said, K/V from three
+// rotating sets): B16 H16 KV 1024-4096 pages of 16 125 -> 59-68 us, B8 H32 KV 2048
+// D 96 65 -> 33 us, D 64 KV 4096 pages of 16 96 -> 53 us, D 256 B8 H8 KV 2048 31.6
+// -> 25.5 us, B4 H32 KV 512 10.8 -> 9.8 us, B1 H1 KV 512 8.2 -> 7.8 us. Steps of 32
+// keys at D 128 (twice the registers, one workgroup per CU) measured 0-8% slower
+// except on the shortest calls (B1 H1 KV 512 7.4 us); 4 waves 1-7% slower; the heads
+// of a key range as neighbours instead of a head's splits 7% slower.
 #pragma once
 #include "fmha_kernel.h"
 
@@ -373,7 +374,7 @@ __global__ __launch_bounds__(C::THREADS, 4) void decode_kernel(FwdParams p_arg,
     for (int j = 0; j < 8; ++j) st.acc[j] = 0.0f;
     if (n < it.end) {
       if (n != guess) ids = step_ids<C>(p, it.table_b, n, lane);
-      if (non_temporal_kv(p, len, row_bytes))
+      if (stream_kv(p, stream_probe(p, table, lengths, b, (n - wave) * C::STEP, lane), row_bytes, lane))
         decode_steps<C, true>(p, it, n, ids, q, st, lane, lane_off);
       else
         decode_steps<C, false>(p, it, n, ids, q, st, lane, lane_off);

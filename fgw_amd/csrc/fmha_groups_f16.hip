@@ -1,9 +1,10 @@
-// F16 instantiations of the key and query layouts' row-group kernels and of the
-// query layout's eight-wave kernel.
+// F16 instantiations of the key and query layouts' row-group kernels, of
+// the key layout's with non-temporal loads and of the query layout's eight-wave one.
 #include "fmha_kernel.h"
 #include "fmha_registry.h"
 
 namespace fgw_mha {
 FGW_MHA_FOR_GROUPS(FGW_MHA_INSTANTIATE_GROUPS, false)
+FGW_MHA_FOR_STREAM(FGW_MHA_INSTANTIATE_STREAM, false)
 FGW_MHA_INSTANTIATE_DUAL(false)
 }  // namespace fgw_mha

@@ -58,6 +58,8 @@
 // the program id so that neighbouring items share an XCD's L2.
 #pragma once
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 #include <stdint.h>
 
 #include "fmha_params.h"
@@ -171,26 +173,6 @@ __device__ __forceinline__ ProgramItems key_items(int work) {
   return ProgramItems{a + local, nx, local < end - a ? (end - a - local + nx - 1) / nx : 0};
 }
 
-// Whether a work item (key and query layouts) loads K/V non-temporally: nothing
-// else of the call reads its rows again (one query tile, and head rows that
-// fill whole 128-byte lines, which heads would otherwise share), and a batch
-// of requests of its length is too large for the 256 MB last-level cache to
-// keep until the next call. Large reads then gain what the cache's
-// allocations cost; below that size repeated calls find their K/V there.
-// Measured over three rotating sets of inputs, the time non-temporal over
-// plain: B8 H8 D128 KV 512 / 1024 / 2048 (16 / 32 / 64 MiB) 1.20 / 1.29 /
-// 1.07, KV 3072 (96 MiB) 0.99, KV 4096-8192 (128-256 MiB) 0.89-0.90; D 16 and
-// 48 (shared lines) 1.45 and 1.11; two query tiles 1.21. The price: a program that
-// repeats one call on one set of 128-256 MiB, with nothing in between, no longer
-// finds part of it in that cache (B2 H8 KV 32768, 256 MiB, the same call back to
-// back 43.7 -> 45.9 us; on rotating sets 53.7 -> 46.7). A decode loop reads the
-// other layers' K/V between two steps of one layer, so the second is its case.
-constexpr int64_t kNonTemporalBytes = int64_t(128) << 20;
-__device__ __forceinline__ bool non_temporal_kv(const FwdParams& p, int len, int64_t row_bytes) {
-  return p.q_tiles == 1 && p.dim % 64 == 0 &&
-         2 * (int64_t)len * p.batch * row_bytes >= kNonTemporalBytes;
-}
-
 template <int A, int B>
 struct CMax {
   static constexpr int value = A > B ? A : B;
@@ -202,7 +184,9 @@ struct CMin {
 
 // Variants of fwd_kernel.
 // kGroups: the page table is resolved per DMA instruction instead of per block
-// (GroupRows).
+// (GroupRows); non-temporal loads where stream_kv says so.
+// kStream (key layout): the plain kernel with non-temporal loads where stream_kv
+// says so, for table capacities that can exceed the last-level cache.
 // kDual (query layout, head-dim tile 256): two sets of four waves hold the same
 // 128 query rows, each takes 32 keys of every 64-key block, and their states
 // meet in LDS at the end of an item. At this tile the K/V stages fill a CU's LDS
@@ -214,12 +198,13 @@ struct CMin {
 // us, B2 H8 Q1024 KV 2048 causal 59.8 / 55.2 us. Which plans take it: dual_takes
 // (fmha_api.hip). With padded head dims and small pages (row groups) the same
 // split measured 0.73 to 1.08 of the plain kernel's speed, and is not built.
-enum Variant : int { kPlain = 0, kGroups = 1, kDual = 2 };
+enum Variant : int { kPlain = 0, kGroups = 1, kDual = 2, kStream = 3 };
 template <bool BF16_, int DPAD_, int LAYOUT_, int STAGES_ = 0, int VARIANT_ = kPlain>
 struct Cfg {
   static constexpr bool BF16 = BF16_;
   static constexpr int VARIANT = VARIANT_;
   static constexpr bool GROUPS = VARIANT == kGroups;
+  static constexpr bool STREAM = VARIANT == kStream;
   static constexpr int DPAD = DPAD_;  // head dim padded to a power of two >= 32
   static constexpr int LAYOUT = LAYOUT_;
   static constexpr int NWQ = LAYOUT == kLayoutQuery ? 4 : 1;  // waves along queries
@@ -383,14 +368,59 @@ struct DmaLanes {
   __device__ __forceinline__ u32 vq(int q, int wq) const { return PRE ? voff[PRE ? q : 0] : v(q, wq); }
 };
 
+// Whether a work item's K/V loads are non-temporal, that is, pass by the 256 MB
+// last-level cache. p.stream_bytes is the host's limit (stream_bytes_of in
+// fmha_api.hip; 0: never): above it a call's live K/V are worth more read past
+// the cache than kept in it. They are the sum of the live lengths (of the next 64
+// requests for a larger batch, scaled), and not more than the pool. An item
+// whose first page another of the next 64 requests has at the same place of
+// its table (a common prefix) keeps the cached loads: the other requests' items
+// read those rows again. Shared prefixes, BF16 D128, non-temporal loads on every
+// item / by this rule / no such loads at all: B32 H8 Sq 1 KV 8192 114 / 71.2 / 69.8
+// us, B64 H8 Sq 8 KV 4096 111 / 73.5 / 71.9, B16 H16 Sq 1 KV 16384 275 / 152 / 153.
+// In two parts, so that a kernel can have the loads of the first in flight.
+struct StreamProbe {
+  int32_t own, other, len;  // page ids of b and of the lane's request, its length
+};
+__device__ __forceinline__ StreamProbe stream_probe(const FwdParams& p, const int32_t* table,
+                                                    const int32_t* lengths, int b, int pos,
+                                                    int lane) {
+  if (p.stream_bytes == 0) return StreamProbe{0, 0, 0};
+  u32 pg = div_page((u32)pos, p.page_magic, p.page_shift);
+  pg = pg < (u32)p.width ? pg : (u32)p.width - 1u;
+  const int ahead = opaque_lane(lane) + 1;  // of the requests after b, cyclically
+  int other = ahead < p.batch ? b + ahead : b;
+  other -= other >= p.batch ? p.batch : 0;
+  return StreamProbe{table[(int64_t)b * p.width + pg], table[(int64_t)other * p.width + pg],
+                     lengths[other]};
+}
+__device__ __forceinline__ bool stream_kv(const FwdParams& p, const StreamProbe& probe,
+                                          int64_t row_bytes, int lane) {
+  if (p.stream_bytes == 0) return false;
+  lane = opaque_lane(lane);
+  const int capacity = p.width * p.page_size;
+  const bool another = lane + 1 < p.batch;
+  if (__ballot(another && probe.other == probe.own) != 0) return false;
+  const int len = probe.len < 0 ? 0 : (probe.len > capacity ? capacity : probe.len);
+  // (Lanes without another request hold b's own length: one of them counts.)
+  float rows = another || lane + 1 == p.batch ? (float)len : 0.0f;
+#pragma unroll
+  for (int x = 1; x < 64; x *= 2)
+    rows += __uint_as_float((u32)__builtin_amdgcn_ds_bpermute(4 * (lane ^ x),
+                                                              (int)__float_as_uint(rows)));
+  if (p.batch > 64) rows *= (float)p.batch * 0.015625f;
+  rows = fminf(rows, (float)p.pool_rows);
+  return 2.0f * rows * (float)row_bytes > (float)p.stream_bytes;
+}
+
 // Issue the DMA loads of the K (IS_V false) or V tile of keys
 // [pos0, pos0 + BN) of (b, h) into LDS at `dst`. Wave `wq` of the key group
 // issues the instructions i = q * NWQ + wq. `id0` is the page id of the page
 // holding pos0 (read ahead by the caller). A block inside one page, below
 // len, with no padded dims takes the fast path: uniform row base + per-lane
-// offset. Otherwise every key is resolved through the table and masked
-// chunks read the zero chunk.
-template <class C, bool IS_V>
+// offset (NT: non-temporal). Otherwise every key is resolved through the table
+// and masked chunks read the zero chunk.
+template <class C, bool IS_V, bool NT = false>
 __device__ __forceinline__ void issue_tile(const FwdParams& p, const DmaLanes<C>& dl,
                                            const int32_t* table_b, const char* base,
                                            int64_t row_bytes, int pos0, int32_t id0, int len,
@@ -417,7 +447,8 @@ __device__ __forceinline__ void issue_tile(const FwdParams& p, const DmaLanes<C>
         dma_saddr(base + rb, off, dst + 1024u * i);
       else
         __builtin_amdgcn_global_load_lds(base + rb + off,
-                                         FGW_LDS(void, (uintptr_t)(dst + 1024u * i)), 16, 0, 0);
+                                         FGW_LDS(void, (uintptr_t)(dst + 1024u * i)), 16, 0,
+                                         NT ? 2 : 0);
     }
     return;
   }
@@ -1353,13 +1384,18 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
     const int first_pos = tile_of(blk_begin);
     const bool spec = first_pos == spec_pos;
     if (it > 0) __syncthreads();  // LDS of the previous work item is no longer read
-    // Every key group streams its blocks n = 0, 1, ... at key
-    // (blk_begin + wk + NWK n) * BN through its own LDS stages; the DMA of
-    // block n + 1 is in flight while block n is computed.
+    // Every key group streams its tiles n = 0, 1, ... at key first_pos + kStep n
+    // through its own LDS stages; the DMA of tile n + 1 is in flight while tile n
+    // is computed.
     int32_t next_id = my_n > 1 ? (spec ? spec1 : ids_of(first_pos + kStep)) : 0;
-    const bool nt = C::GROUPS && non_temporal_kv(p, len, row_bytes);
+    // Non-temporal loads; kStream decides with its first tile and Q on the way.
+    bool nt = false;
+    StreamProbe probe{0, 0, 0};
+    if constexpr (C::GROUPS || C::STREAM)
+      probe = stream_probe(p, table, lengths, b, blk_begin * C::BLOCK, lane);
+    if constexpr (C::GROUPS) nt = stream_kv(p, probe, row_bytes, lane);
     // K and V of the block at pos (its page ids: id) into a stage.
-    auto issue = [&](int pos, int32_t id, unsigned char* stage) {
+    auto issue = [&](int pos, int32_t id, unsigned char* stage, auto stream) {
       if constexpr (C::GROUPS) {
         const GroupRows g = group_rows<C>(p, row_bytes, pos, id, len, wq, lane);
         if (nt)
@@ -1367,12 +1403,13 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
         else
           issue_groups<C, false>(p, dl, kb, vb, g, stage, wq, lane);
       } else {
-        issue_tile<C, false>(p, dl, table_b, kb, row_bytes, pos, id, len, stage, wq, lane);
-        issue_tile<C, true>(p, dl, table_b, vb, row_bytes, pos, id, len, stage + C::TILE_BYTES, wq,
-                            lane);
+        constexpr bool NT = decltype(stream)::value;
+        issue_tile<C, false, NT>(p, dl, table_b, kb, row_bytes, pos, id, len, stage, wq, lane);
+        issue_tile<C, true, NT>(p, dl, table_b, vb, row_bytes, pos, id, len, stage + C::TILE_BYTES,
+                                wq, lane);
       }
     };
-    if (my_n > 0) issue(first_pos, spec ? spec0 : ids_of(first_pos), group_base);
+    if (my_n > 0) issue(first_pos, spec ? spec0 : ids_of(first_pos), group_base, std::false_type{});
     // Q after the first DMA: its loads overlap the tile's.
     u32x4 qf[C::KK];
     {
@@ -1387,25 +1424,37 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
         qf[kk] = val;
       }
     }
-    for (int n = 0; n < my_n; ++n) {
-      const int pos0 = first_pos + kStep * n;
-      unsigned char* stage = group_base + (n % C::NBUF) * C::STAGE_BYTES;
-      wait_dma();
-      group_sync<C>();  // stage n is in LDS; everyone is done with stage n - 1
-      const int32_t id1 = next_id;
-      if (n + 2 < my_n) next_id = ids_of(pos0 + 2 * kStep);
-      if (n + 1 < my_n && C::NBUF == 2)
-        issue(pos0 + kStep, id1, group_base + ((n + 1) % C::NBUF) * C::STAGE_BYTES);
-      f32x16 s[C::ST];
-      u32x4 pf[C::KS];
-      qk_block<C>(stage, ln, qf, s);
-      if (pos0 + C::BN > wmin) mask_block<C>(s, pos0, vis, hh);
-      online_softmax<C>(s, m, l, o, p.scale_log2, pf);
-      pv_block<C>(stage + C::TILE_BYTES, ln, pf, o);
-      if (n + 1 < my_n && C::NBUF == 1) {
-        group_sync<C>();  // single stage: refill only after every wave has read it
-        issue(pos0 + kStep, id1, stage);
+    // The main loop; stream: its loads are non-temporal (kStream: one loop for each
+    // kind, since a branch in the loop cost 4% on shared pages).
+    auto blocks = [&](auto stream) {
+      for (int n = 0; n < my_n; ++n) {
+        const int pos0 = first_pos + kStep * n;
+        unsigned char* stage = group_base + (n % C::NBUF) * C::STAGE_BYTES;
+        wait_dma();
+        group_sync<C>();  // stage n is in LDS; everyone is done with stage n - 1
+        const int32_t id1 = next_id;
+        if (n + 2 < my_n) next_id = ids_of(pos0 + 2 * kStep);
+        if (n + 1 < my_n && C::NBUF == 2)
+          issue(pos0 + kStep, id1, group_base + ((n + 1) % C::NBUF) * C::STAGE_BYTES, stream);
+        f32x16 s[C::ST];
+        u32x4 pf[C::KS];
+        qk_block<C>(stage, ln, qf, s);
+        if (pos0 + C::BN > wmin) mask_block<C>(s, pos0, vis, hh);
+        online_softmax<C>(s, m, l, o, p.scale_log2, pf);
+        pv_block<C>(stage + C::TILE_BYTES, ln, pf, o);
+        if (n + 1 < my_n && C::NBUF == 1) {
+          group_sync<C>();  // single stage: refill only after every wave has read it
+          issue(pos0 + kStep, id1, stage, stream);
+        }
       }
+    };
+    if constexpr (C::STREAM) {
+      if (stream_kv(p, probe, row_bytes, lane))
+        blocks(std::true_type{});
+      else
+        blocks(std::false_type{});
+    } else {
+      blocks(std::false_type{});
     }
 
     wait_dma();  // no DMA of this work item outlives it

@@ -13,6 +13,7 @@ enum Kernel : int32_t {
   kKernelQueryDual,      // its eight-wave variant (head-dim tile 256)
   kKernelKey,            // fwd_kernel, key layout
   kKernelKeyGroups,      // its row-group variant
+  kKernelKeyStream,      // its variant with non-temporal loads
   kKernelDecode,         // decode_kernel (Sq = 1)
   kKernelPrefill,        // prefill_kernel
   kKernelPrefillGroups,  // its row-group variant
@@ -28,6 +29,7 @@ struct LaunchInfo {
   int32_t q_tiles;        // ceil(Sq / rows of its query tiles)
   int32_t work_items;
   int32_t grid;           // programs
+  int64_t stream_bytes;   // FwdParams::stream_bytes
 };
 
 }  // namespace fgw_mha

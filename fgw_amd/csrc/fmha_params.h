@@ -49,6 +49,9 @@ struct FwdParams {
   // Tile-balanced plans in a whole call: a tile of one split writes its
   // normalised output rows directly (the merge skips them).
   int32_t split_direct;
+  // Live K/V bytes above which a work item's loads are non-temporal (stream_kv in
+  // fmha_kernel.h); 0: never.
+  int64_t stream_bytes;
   // Fused split merge (mode 1, query and key layouts): one counter per task
   // (b H + h) q_tiles + q tile, zero on entry; every work item counts itself
   // in once its partial rows are written, the last one of a task merges the

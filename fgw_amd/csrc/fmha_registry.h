@@ -29,6 +29,9 @@ FwdEntry fwd_entry(bool bf16, int dpad, int layout, int stages = 0);
 FwdLaunchFn prefill_rows_entry(bool bf16, int dpad, int rows);
 // The row-group kernel of (dtype, head-dim tile, key or query layout, stages).
 FwdLaunchFn groups_entry(bool bf16, int dpad, int layout, int stages);
+// The key layout's kernel with non-temporal loads (kStream) of (dtype, head-dim
+// tile, stages); null for tile 32.
+FwdLaunchFn stream_entry(bool bf16, int dpad, int stages);
 // The query layout's kernel of eight waves (kDual), head-dim tile 256.
 FwdLaunchFn dual_entry(bool bf16);
 // The half-tile kernel of (dtype, head-dim tile, rows mode).
@@ -83,6 +86,13 @@ hipError_t launch_group_merge(bool bf16, const GroupMergeParams& p, int groups, 
   template hipError_t launch_fwd<BF, DP, LY, ST, kGroups>(const FwdParams&, int, hipStream_t);
 #define FGW_MHA_EXTERN_GROUPS(BF, DP, LY, ST) \
   extern template hipError_t launch_fwd<BF, DP, LY, ST, kGroups>(const FwdParams&, int, hipStream_t);
+// The key layout's kernels with non-temporal loads.
+#define FGW_MHA_FOR_STREAM(X, BF) X(BF, 64, 0) X(BF, 128, 0) X(BF, 256, 0) X(BF, 128, 1)
+#define FGW_MHA_INSTANTIATE_STREAM(BF, DP, ST) \
+  template hipError_t launch_fwd<BF, DP, kLayoutKey, ST, kStream>(const FwdParams&, int, hipStream_t);
+#define FGW_MHA_EXTERN_STREAM(BF, DP, ST) \
+  extern template hipError_t launch_fwd<BF, DP, kLayoutKey, ST, kStream>(const FwdParams&, int, \
+                                                                         hipStream_t);
 // The query layout's eight-wave kernel, head-dim tile 256.
 #define FGW_MHA_INSTANTIATE_DUAL(BF) \
   template hipError_t launch_fwd<BF, 256, kLayoutQuery, 0, kDual>(const FwdParams&, int, hipStream_t);

@@ -69,8 +69,11 @@ def test_both_stage_counts_and_ids_outside_the_pool(stages):
 def test_length_balanced_and_non_temporal():
     _check(70, 2, 1, 64, 16, [(29 * i) % 400 for i in range(70)], torch.float16, num_splits=4,
            split_keys=128, kernel="key_groups")
-    # 2 x 40 x 4096 x 8 x 64 x 2 bytes = 168 MB of K/V.
-    _check(40, 2, 8, 64, 128, [4096 - 31 * i for i in range(40)], torch.float16, num_splits=1)
+    # 4 x 40 x 4096 x 8 x 64 bytes = 320 MiB of K/V, 272 MiB live; with pages of 16, 168 of 192.
+    _check(40, 2, 8, 64, 128, [4096 - 31 * i for i in range(40)], torch.float16, num_splits=1,
+           kernel="key_stream")
+    _check(24, 2, 8, 64, 16, [4096 - 41 * i for i in range(24)], torch.float16, num_splits=1,
+           kernel="key_groups")
 
 
 @gpu

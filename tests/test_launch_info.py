@@ -38,6 +38,39 @@ def test_variant_of_a_plan(name, kwargs):
         assert (info.q_tiles, info.work_items, info.grid) == (plan.q_tiles, plan.work_items, plan.grid)
 
 
+MIB = 1 << 20
+
+
+@pytest.mark.parametrize("name,stream,kwargs", [
+    # Whole blocks at tile 128: the key kernel from 128 MiB of K/V, past the cache above 256.
+    ("decode", 0, dict(kv=16383 // 64 * 64)), ("key", 0, dict(kv=16384)), ("key", 0, dict(kv=32768)),
+    ("key_stream", 256, dict(kv=32832)), ("key_stream", 256, dict(sq=8, kv=32832)),
+    ("key", 0, dict(sq=8, kv=32768)),
+    # Tile 64: the single-token kernel below the cache's size.
+    ("decode", 0, dict(d=64, kv=65472)), ("key", 0, dict(d=64, kv=65536)),
+    ("key_stream", 256, dict(d=64, kv=65600)),
+    # Small pages, padded head dims and D 256: the same kernel at any size, past the
+    # cache from half of it.
+    ("decode", 0, dict(page=16, kv=16384)), ("decode", 128, dict(page=16, kv=16400)),
+    ("decode", 128, dict(d=192, kv=65536)), ("decode", 128, dict(d=256, kv=65536)),
+    ("key_groups", 128, dict(sq=8, page=16, kv=16400)),
+    # Heads that share 128-byte lines, and more than one query tile: never.
+    ("decode", 0, dict(d=80, kv=65536)), ("key_groups", 0, dict(sq=8, d=96, kv=65536)),
+    ("query_groups", 128, dict(sq=128, page=16, kv=32768, layout=0)),
+    ("query_groups", 0, dict(sq=129, page=16, kv=32768, layout=0))])
+def test_large_caches(name, stream, kwargs):
+    _, info = launch(**kwargs)
+    assert (info.name, info.stream_bytes) == (name, stream * MIB)
+
+
+def test_a_shared_pool_is_not_counted_per_request():
+    """64 requests that share 8192 rows: 32 MiB of K/V fit the cache, 2 GiB are read from it."""
+    shape = _lib.Shape(64, 1, 8, 128, 8192, 128, 64, 0, _lib.DTYPE_BFLOAT16)
+    plan = _lib.plan(shape, _lib.Request(0, -1, -1), DEVICE)
+    info = _lib.launch_info(shape, plan)
+    assert (info.name, info.stream_bytes) == ("key", 0)
+
+
 def test_a_plan_of_another_shape_is_refused():
     plan, _ = launch()
     other = _lib.Shape(3, 1, 8, 128, 4096, 32, 64, 0, _lib.DTYPE_BFLOAT16)
