@@ -889,6 +889,8 @@ int fgw_mha_plan(const fgw_mha_shape* s, const fgw_mha_request* req,
                            ? tile_balanced_work(s, splits, split_keys)
                            : tasks * splits;
   if (work > INT32_MAX) return fail(FGW_MHA_EUNSUPPORTED, "work items exceed 2^31");
+  if (req->persistent_programs < -1)
+    return fail(FGW_MHA_EINVAL, "persistent_programs must be -1, 0 or positive");
 
   // Stages: the layout's default kernel unless the request names one or the
   // automatic splits moved to the key layout's single-stage kernel (head-dim
@@ -898,13 +900,27 @@ int fgw_mha_plan(const fgw_mha_shape* s, const fgw_mha_request* req,
   // few ways (B8 H32 KV 4096, 2 splits: 115.9 us against 101.7 us at 1 split).
   const int stages =
       req->stages != 0 ? req->stages : (auto_single ? 1 : default_stages(layout, dpad));
-  const int wg_kernel = stages == 1 && has_key_single(layout, dpad)
-                            ? (dev->wg_per_cu_key_single > 0 ? dev->wg_per_cu_key_single : 1)
-                            : wg_default;
+  out->layout = layout;
+  out->rows_per_tile = rows;
+  out->q_tiles = q_tiles;
+  out->num_splits = splits;
+  out->query_tile_tasks = (int32_t)tasks;
+  out->work_items = (int32_t)work;
+  out->threads = layout == kLayoutPrefill ? 512 : 256;
+  out->execution_mode = splits > 1 ? 1 : 0;
+  out->dim_padded = dpad;
+  out->parts_floats = splits > 1 ? (int64_t)s->batch * s->heads * splits * s->sq * s->dim : 0;
+  out->lse_floats = splits > 1 ? (int64_t)s->batch * s->heads * splits * s->sq : 0;
+  out->split_keys = split_keys;
+  out->stages = stages;
+  // The selected kernel's resident workgroups. A stage count asked for keeps the
+  // residency of the key kernel that it names.
+  const int wg_single = dev->wg_per_cu_key_single > 0 ? dev->wg_per_cu_key_single : 1;
+  const bool decode = req->stages == 0 && kernel_of(s, out) == kKernelDecode;
+  const int wg_kernel = decode ? kDecodeWgPerCu
+                        : stages == 1 && has_key_single(layout, dpad) ? wg_single : wg_default;
 
   int64_t grid = work;
-  if (req->persistent_programs < -1)
-    return fail(FGW_MHA_EINVAL, "persistent_programs must be -1, 0 or positive");
   if (req->persistent_programs == -1 && !s->causal) {
     // Device cap: the resident workgroups of all CUs loop over contiguous
     // ranges of work items. Causal work items differ in size (and with
@@ -916,21 +932,7 @@ int fgw_mha_plan(const fgw_mha_shape* s, const fgw_mha_request* req,
   } else if (req->persistent_programs > 0) {
     grid = work < req->persistent_programs ? work : req->persistent_programs;
   }
-
-  out->layout = layout;
-  out->rows_per_tile = rows;
-  out->q_tiles = q_tiles;
-  out->num_splits = splits;
-  out->query_tile_tasks = (int32_t)tasks;
-  out->work_items = (int32_t)work;
   out->grid = (int32_t)grid;
-  out->threads = layout == kLayoutPrefill ? 512 : 256;
-  out->execution_mode = splits > 1 ? 1 : 0;
-  out->dim_padded = dpad;
-  out->parts_floats = splits > 1 ? (int64_t)s->batch * s->heads * splits * s->sq * s->dim : 0;
-  out->lse_floats = splits > 1 ? (int64_t)s->batch * s->heads * splits * s->sq : 0;
-  out->split_keys = split_keys;
-  out->stages = stages;
   out->arrival_counters = (int32_t)fused_merge_counters(s, layout, splits, rows, tasks);
   return FGW_MHA_OK;
 }

@@ -15,10 +15,10 @@ def lib():
 
 
 def launch(b=2, sq=1, h=8, d=128, kv=2048, page=64, causal=0, layout=-1, splits=0, programs=-1,
-           split_keys=0):
+           split_keys=0, stages=0):
     width = -(-kv // page)
     shape = _lib.Shape(b, sq, h, d, b * width * page, width, page, causal, _lib.DTYPE_BFLOAT16)
-    plan = _lib.plan(shape, _lib.Request(splits, programs, layout, split_keys), DEVICE)
+    plan = _lib.plan(shape, _lib.Request(splits, programs, layout, split_keys, stages), DEVICE)
     return plan, _lib.launch_info(shape, plan)
 
 
@@ -69,6 +69,16 @@ def test_a_shared_pool_is_not_counted_per_request():
     plan = _lib.plan(shape, _lib.Request(0, -1, -1), DEVICE)
     info = _lib.launch_info(shape, plan)
     assert (info.name, info.stream_bytes) == ("key", 0)
+
+
+def test_device_cap_is_the_selected_kernels_residency():
+    """Two single-token programs per CU; one of the double-stage key kernel's."""
+    assert launch(b=64, h=32, kv=512)[0].grid == 512
+    assert launch(b=64, h=32, kv=512, d=64)[0].grid == 512
+    assert launch(b=64, h=32, kv=512, page=6)[0].grid == 256  # the key kernel
+    assert launch(b=64, h=32, kv=512, stages=2)[0].grid == 256  # asked for
+    assert launch(b=64, h=32, kv=512, programs=0)[0].grid == 2048
+    assert launch(b=64, h=32, kv=512, programs=300)[0].grid == 300
 
 
 def test_a_plan_of_another_shape_is_refused():
