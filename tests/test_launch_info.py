@@ -73,12 +73,12 @@ def test_a_shared_pool_is_not_counted_per_request():
 
 def test_device_cap_is_the_selected_kernels_residency():
     """Two single-token programs per CU; one of the double-stage key kernel's."""
-    assert launch(b=64, h=32, kv=512)[0].grid == 512
-    assert launch(b=64, h=32, kv=512, d=64)[0].grid == 512
-    assert launch(b=64, h=32, kv=512, page=6)[0].grid == 256  # the key kernel
-    assert launch(b=64, h=32, kv=512, stages=2)[0].grid == 256  # asked for
-    assert launch(b=64, h=32, kv=512, programs=0)[0].grid == 2048
-    assert launch(b=64, h=32, kv=512, programs=300)[0].grid == 300
+    assert launch(b=64, h=32, kv=64)[0].grid == 512
+    assert launch(b=64, h=32, kv=256, d=64)[0].grid == 512
+    assert launch(b=64, h=32, kv=64, page=6)[0].grid == 256  # the key kernel
+    assert launch(b=64, h=32, kv=64, stages=2)[0].grid == 256  # asked for
+    assert launch(b=64, h=32, kv=64, programs=0)[0].grid == 2048
+    assert launch(b=64, h=32, kv=64, programs=300)[0].grid == 300
 
 
 def test_a_plan_of_another_shape_is_refused():
