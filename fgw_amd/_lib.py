@@ -69,7 +69,7 @@ KERNELS = ("query", "query_groups", "query_eight_waves", "key", "key_groups", "k
 class LaunchInfo(ctypes.Structure):
     _fields_ = [("kernel", c_int32), ("threads", c_int32), ("rows_per_item", c_int32),
                 ("q_tiles", c_int32), ("work_items", c_int32), ("grid", c_int32),
-                ("stream_bytes", c_int64)]
+                ("stream_bytes", c_int64), ("longest_first", c_int32)]
 
     @property
     def name(self) -> str:

@@ -501,6 +501,7 @@ FwdParams make_params(const fgw_mha_shape* s, const fgw_mha_plan_t* p, const fgw
   f.split_keys = mode == 1 ? p->split_keys : 0;
   f.split_direct = 0;
   f.stream_bytes = 0;
+  f.longest_first = 0;
   page_divisor((uint32_t)s->page_size, &f.page_magic, &f.page_shift);
   f.scale_log2 = (float)(1.4426950408889634 / __builtin_sqrt((double)s->dim));
   f.segs = nullptr;
@@ -699,6 +700,30 @@ FwdLaunchFn launch_fn(const fgw_mha_shape* s, const fgw_mha_plan_t* p, Kernel ke
   }
 }
 
+// Whether a causal prefill-layout plan takes its items longest first over all (b, h)
+// instead of (b, h) after (b, h). Items differ in length by up to Sq keys; in the
+// order of (b, h) the long tiles of the last ones start last. But neighbours then
+// share an XCD's L2, which the other order gives up: every tile reads its K/V from
+// memory. With `rounds` items of 256 rows per CU, the gain falls with the rounds
+// and with how little Sq is of a mean item's keys (capacity - Sq / 2), and head-dim
+// tile 64, whose items wait for memory less, keeps it longer. Ratios of longest
+// first to (b, h) order over 330 shapes of capacity 2048-16384, tile 64 / 128:
+// capacity = Sq 0.65-0.98 / 0.69-1.0 at 1 to 4 rounds; 2 Sq 0.73-0.97 / 0.76-0.99 up
+// to 3 rounds / 2.5, 0.94-0.98 / 0.96-1.04 at 4; 3 Sq 0.87-1.0 / 0.90-1.01 up to 1.5
+// rounds, 0.96-1.05 / 0.97-1.08 from 2 on; 4 Sq 0.86-0.97 up to 1.75 / 0.88-0.95 up
+// to 1.25, 0.93-1.04 / 0.96-1.13 above; 6 to 32 Sq 0.92-1.01 up to 1.75 / 0.94-1.03
+// up to 1.25, 0.97-1.12 / 0.97-1.16 above. Not below one round, where every item
+// starts at once (256 items of D 64 measured 1.02), nor for single tiles.
+bool longest_first_of(const fgw_mha_shape* s, const fgw_mha_plan_t* p, int work, int rows,
+                      int q_tiles) {
+  if (p->layout != kLayoutPrefill || !s->causal || work <= kNumCus || q_tiles == 1) return false;
+  const bool narrow = p->dim_padded == 64;
+  const int64_t capacity = (int64_t)s->width * s->page_size;
+  const int64_t tiles = (int64_t)work * rows / 256;  // rounds = tiles / kNumCus
+  return 4 * tiles <= (narrow ? 7 : 5) * kNumCus ||
+         (narrow ? 9 : 8) * (int64_t)kNumCus * s->sq >= tiles * (2 * capacity - s->sq);
+}
+
 // What a call of this plan launches. The half-tile kernel's items are half the
 // plan's query tiles, so that it has its own count of them; a plan with fewer
 // programs than items keeps its grid.
@@ -712,6 +737,7 @@ LaunchInfo launch_info(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
   i.rows_per_item = i.kernel == kKernelDecode ? 1 : (half ? kRowsHalfTile : p->rows_per_tile);
   i.q_tiles = half ? (s->sq + kRowsHalfTile - 1) / kRowsHalfTile : p->q_tiles;
   i.work_items = half ? s->batch * s->heads * i.q_tiles : p->work_items;
+  i.longest_first = longest_first_of(s, p, i.work_items, i.rows_per_item, i.q_tiles);
   i.grid = p->grid == p->work_items || p->grid > i.work_items ? i.work_items : p->grid;
   return i;
 }
@@ -726,6 +752,7 @@ int launch_partial_kernel(const fgw_mha_shape* s, const fgw_mha_plan_t* p,
   if (!launch) return fail(FGW_MHA_EUNSUPPORTED, "no kernel for dim tile %d", p->dim_padded);
   FwdParams f = make_params(s, p, t, mode);
   f.stream_bytes = info.stream_bytes;
+  f.longest_first = info.longest_first;
   f.q_tiles = info.q_tiles;
   f.work = info.work_items;
   f.split_direct = whole && mode == 1 && tile_balanced(p->layout, s->causal, p->split_keys);

@@ -74,10 +74,9 @@ __global__ __launch_bounds__(C::THREADS) void half_kernel(FwdParams p_arg,
   const RowDma<C> rd(dl, p.dim, wave, lane);
 
   // Work items in the orders of prefill_kernel: one XCD's programs share a
-  // contiguous, interleaved range; causal items that outnumber the CUs go
-  // longest first over all (b, h).
+  // contiguous, interleaved range, or the items go longest first over all (b, h).
   const int grid = gridDim.x;
-  const bool longest_first = p.causal && p.work > kNumCus;
+  const bool longest_first = p.longest_first != 0;
   ProgramItems items = key_items(p.work);
   if (longest_first)
     items = ProgramItems{(int)blockIdx.x, grid,

@@ -30,6 +30,7 @@ struct LaunchInfo {
   int32_t work_items;
   int32_t grid;           // programs
   int64_t stream_bytes;   // FwdParams::stream_bytes
+  int32_t longest_first;  // FwdParams::longest_first
 };
 
 }  // namespace fgw_mha

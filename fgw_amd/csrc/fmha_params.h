@@ -52,6 +52,8 @@ struct FwdParams {
   // Live K/V bytes above which a work item's loads are non-temporal (stream_kv in
   // fmha_kernel.h); 0: never.
   int64_t stream_bytes;
+  // Prefill layout, causal: work items longest first over all (b, h).
+  int32_t longest_first;
   // Fused split merge (mode 1, query and key layouts): one counter per task
   // (b H + h) q_tiles + q tile, zero on entry; every work item counts itself
   // in once its partial rows are written, the last one of a task merges the

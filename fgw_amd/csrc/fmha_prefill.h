@@ -449,15 +449,10 @@ __global__ __launch_bounds__(C::THREADS) void prefill_kernel(FwdParams p_arg,
   const int per = p.work / grid, rem = p.work % grid;
   const int a = sx * per + (sx < rem ? sx : rem);
   const int end = (sx + nx) * per + (sx + nx < rem ? sx + nx : rem);
-  // Causal items differ in length. Where there are more of them than CUs they
-  // are taken longest first over all (b, h), in dispatch order, so that every
-  // XCD has its share of each length and its CUs fill up with the short ones;
-  // with the tiles of one (b, h) after the other, the long tiles of the last
-  // (b, h) started last. Measured (one split): B1 H32 S4096 D64 124 -> 87 us,
-  // D128 168 -> 131 us, B4 H32 S2048 D128 186 -> 165 us. Fewer items all start
-  // at once, and keep the order whose neighbours share an XCD's L2 (the other
-  // order measured 2% slower at 256 items of D64).
-  const bool longest_first = p.causal && p.work > kNumCus;
+  // longest_first: the items of every (b, h) by length instead, in dispatch order,
+  // so that every XCD has its share of each length and its CUs fill up with the
+  // short ones (longest_first_of in fmha_api.hip).
+  const bool longest_first = p.longest_first != 0;
   const int first = longest_first ? (int)blockIdx.x : a + local, step = longest_first ? grid : nx;
   const int count = longest_first
                         ? ((int)blockIdx.x < p.work ? (p.work - 1 - (int)blockIdx.x) / grid + 1 : 0)

@@ -95,22 +95,26 @@ def test_page_ids_outside_the_pool_read_as_zeros(d, page):
 
 
 @gpu
-@pytest.mark.parametrize("sq,lengths,plan", [
-    (2049, [2100, 2049], dict(num_splits=1)),                  # 9 tiles x 34 (b, h) > 256 items
-    (1030, [1030, 700], dict(num_splits=2)),                   # split items, Sq > len rows
-    (2049, [2100, 2049], dict(num_splits=4, split_keys=640)),  # tiles of 1 to 4 splits
-    (2049, [2100, 2049], dict(num_splits=1, persistent_programs=40)),
+@pytest.mark.parametrize("h,sq,lengths,first,plan", [
+    (17, 2049, [2100, 2049], 1, dict(num_splits=1)),                  # 9 tiles x 34 (b, h)
+    (17, 1030, [1030, 700], 1, dict(num_splits=2)),                   # Sq > len rows
+    (17, 2049, [2100, 2049], 1, dict(num_splits=4, split_keys=640)),  # tiles of 1 to 4 splits
+    (17, 2049, [2100, 2049], 1, dict(num_splits=1, persistent_programs=40)),
+    (120, 300, [2100, 1000], 0, dict(num_splits=1)),                  # 2 tiles x 240
+    (120, 300, [2100, 1000], 0, dict(num_splits=1, persistent_programs=50)),
 ])
-def test_more_causal_items_than_cus(sq, lengths, plan):
-    """Longest-first order: every item is done once, whatever the plan and grid."""
+def test_more_causal_items_than_cus(h, sq, lengths, first, plan):
+    """Longest first or (b, h) after (b, h): every item is done once, whatever the plan and
+    grid."""
     from fgw_amd.operators.mha.current import build_kernel
-    b, h, d, page = 2, 17, 64, 64
+    b, d, page = 2, 64, 64
     width = -(-max(lengths) // page)
     q, k, v, table = O.make_inputs(("order", b, sq, h, d, page, width), 3, torch.float16)
     lengths = torch.tensor(lengths, dtype=torch.int32)
     kern = build_kernel(b, sq, h, d, k.shape[0], width, page, True, "float16", 0, layout="prefill",
                         **plan)
     assert kern.compute_work > 256 and kern.launch_info.name == "prefill"
+    assert kern.launch_info.longest_first == first
     got = kern(*[x.cuda() for x in (q, k, v, table, lengths)]).cpu()
     rtol, atol = O.TOLERANCES[torch.float16]
     torch.testing.assert_close(got, O.chunked_reference(q, k, v, table, lengths, page, True),

@@ -71,6 +71,24 @@ def test_a_shared_pool_is_not_counted_per_request():
     assert (info.name, info.stream_bytes) == ("key", 0)
 
 
+@pytest.mark.parametrize("first,kwargs", [
+    # Whole prompts, 1.5 to 8 items per CU.
+    (1, dict(b=1, h=32, sq=4096, kv=4096)), (1, dict(b=8, h=32, sq=2048, kv=2048)),
+    # Chunks of a long cache: two items per (b, h) re-read its K/V in the other order.
+    (0, dict(b=8, h=32, sq=512, kv=8192)), (0, dict(b=8, h=32, sq=300, kv=8192)),
+    (0, dict(b=8, h=32, sq=512, kv=8192, d=64)), (0, dict(b=16, h=32, sq=512, kv=2048)),
+    # Little more than one item per CU, and not more than one; single tiles.
+    (1, dict(b=9, h=16, sq=512, kv=8192)), (0, dict(b=8, h=16, sq=512, kv=8192)),
+    (0, dict(b=12, h=16, sq=512, kv=8192)), (1, dict(b=12, h=16, sq=512, kv=8192, d=64)),
+    (0, dict(b=9, h=32, sq=256, kv=2048)),
+    # Half a long table: up to two and a half items per CU.
+    (1, dict(b=5, h=8, sq=4096, kv=8192)), (0, dict(b=8, h=8, sq=4096, kv=8192)),
+    # Not causal, another layout.
+    (0, dict(b=1, h=32, sq=4096, kv=4096, causal=0)), (0, dict(b=1, h=32, sq=4096, kv=4096, d=256))])
+def test_order_of_causal_items(first, kwargs):
+    assert launch(**{"causal": 1, **kwargs})[1].longest_first == first
+
+
 def test_device_cap_is_the_selected_kernels_residency():
     """Two single-token programs per CU; one of the double-stage key kernel's."""
     assert launch(b=64, h=32, kv=64)[0].grid == 512
