@@ -436,6 +436,8 @@ int check_shape(const fgw_mha_shape* s) {
   return FGW_MHA_OK;
 }
 
+int check_grid(const fgw_mha_shape* s, const fgw_mha_plan_t* p);
+
 int check_plan(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
   if (!p) return fail(FGW_MHA_EINVAL, "plan is NULL");
   if (p->layout != kLayoutQuery && p->layout != kLayoutKey && p->layout != kLayoutPrefill)
@@ -450,14 +452,13 @@ int check_plan(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
                            : tasks * p->num_splits;
   if (p->rows_per_tile != rows || p->q_tiles != q_tiles || p->query_tile_tasks != tasks ||
       p->num_splits < 1 || p->num_splits > kMaxSplits || p->work_items != work ||
-      p->grid < 1 || p->grid > p->work_items ||
       p->dim_padded != dim_tile(s->dim) || p->execution_mode != (p->num_splits > 1 ? 1 : 0) ||
       !split_keys_valid(s, p->layout, p->num_splits, p->split_keys) ||
       !stages_valid(p->layout, p->dim_padded, p->stages) ||
       (p->arrival_counters != 0 &&
        p->arrival_counters != fused_merge_counters(s, p->layout, p->num_splits, rows, tasks)))
     return fail(FGW_MHA_EINVAL, "plan does not match the shape; call fgw_mha_plan");
-  return FGW_MHA_OK;
+  return check_grid(s, p);
 }
 
 int check_tensors(const fgw_mha_tensors* t, bool need_inputs, bool need_out, bool need_ws) {
@@ -724,22 +725,38 @@ bool longest_first_of(const fgw_mha_shape* s, const fgw_mha_plan_t* p, int work,
          (narrow ? 9 : 8) * (int64_t)kNumCus * s->sq >= tiles * (2 * capacity - s->sq);
 }
 
-// What a call of this plan launches. The half-tile kernel's items are half the
-// plan's query tiles, so that it has its own count of them; a plan with fewer
-// programs than items keeps its grid.
+bool half_kernel_id(Kernel kernel) { return kernel == kKernelHalf || kernel == kKernelHalfPadded; }
+int half_q_tiles(const fgw_mha_shape* s) { return (s->sq + kRowsHalfTile - 1) / kRowsHalfTile; }
+// Work items of a plan's kernel. The half-tile kernel's are half the plan's query
+// tiles; every other kernel runs the plan's work items.
+int items_of(const fgw_mha_shape* s, const fgw_mha_plan_t* p, Kernel kernel) {
+  return half_kernel_id(kernel) ? s->batch * s->heads * half_q_tiles(s) : p->work_items;
+}
+int threads_of(Kernel kernel, int layout) {
+  return layout == kLayoutPrefill || kernel == kKernelDecode || kernel == kKernelQueryDual ? 512 : 256;
+}
+
+// What a call of this plan launches.
 LaunchInfo launch_info(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
   LaunchInfo i;
-  i.kernel = kernel_of(s, p);
-  i.stream_bytes = stream_bytes_of(s, p, (Kernel)i.kernel);
-  const bool half = i.kernel == kKernelHalf || i.kernel == kKernelHalfPadded;
-  i.threads = p->layout == kLayoutPrefill || i.kernel == kKernelDecode || i.kernel == kKernelQueryDual
-                  ? 512 : 256;
-  i.rows_per_item = i.kernel == kKernelDecode ? 1 : (half ? kRowsHalfTile : p->rows_per_tile);
-  i.q_tiles = half ? (s->sq + kRowsHalfTile - 1) / kRowsHalfTile : p->q_tiles;
-  i.work_items = half ? s->batch * s->heads * i.q_tiles : p->work_items;
+  const Kernel kernel = kernel_of(s, p);
+  const bool half = half_kernel_id(kernel);
+  i.kernel = kernel;
+  i.stream_bytes = stream_bytes_of(s, p, kernel);
+  i.threads = threads_of(kernel, p->layout);
+  i.rows_per_item = kernel == kKernelDecode ? 1 : (half ? kRowsHalfTile : p->rows_per_tile);
+  i.q_tiles = half ? half_q_tiles(s) : p->q_tiles;
+  i.work_items = items_of(s, p, kernel);
   i.longest_first = longest_first_of(s, p, i.work_items, i.rows_per_item, i.q_tiles);
-  i.grid = p->grid == p->work_items || p->grid > i.work_items ? i.work_items : p->grid;
+  i.grid = p->grid < i.work_items ? p->grid : i.work_items;
   return i;
+}
+
+// A plan's grid: not more programs than the kernel has items.
+int check_grid(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
+  if (p->grid < 1 || p->grid > items_of(s, p, kernel_of(s, p)))
+    return fail(FGW_MHA_EINVAL, "plan does not match the shape; call fgw_mha_plan");
+  return FGW_MHA_OK;
 }
 
 // `whole`: the partial kernel of a full call, whose merge follows (a
@@ -933,7 +950,6 @@ int fgw_mha_plan(const fgw_mha_shape* s, const fgw_mha_request* req,
   out->num_splits = splits;
   out->query_tile_tasks = (int32_t)tasks;
   out->work_items = (int32_t)work;
-  out->threads = layout == kLayoutPrefill ? 512 : 256;
   out->execution_mode = splits > 1 ? 1 : 0;
   out->dim_padded = dpad;
   out->parts_floats = splits > 1 ? (int64_t)s->batch * s->heads * splits * s->sq * s->dim : 0;
@@ -943,11 +959,13 @@ int fgw_mha_plan(const fgw_mha_shape* s, const fgw_mha_request* req,
   // The selected kernel's resident workgroups. A stage count asked for keeps the
   // residency of the key kernel that it names.
   const int wg_single = dev->wg_per_cu_key_single > 0 ? dev->wg_per_cu_key_single : 1;
-  const bool decode = req->stages == 0 && kernel_of(s, out) == kKernelDecode;
+  const Kernel kernel = kernel_of(s, out);
+  const bool decode = req->stages == 0 && kernel == kKernelDecode;
   const int wg_kernel = decode ? kDecodeWgPerCu
                         : stages == 1 && has_key_single(layout, dpad) ? wg_single : wg_default;
 
-  int64_t grid = work;
+  const int64_t items = items_of(s, out, kernel);
+  int64_t grid = items;
   if (req->persistent_programs == -1 && !s->causal) {
     // Device cap: the resident workgroups of all CUs loop over contiguous
     // ranges of work items. Causal work items differ in size (and with
@@ -955,11 +973,12 @@ int fgw_mha_plan(const fgw_mha_shape* s, const fgw_mha_request* req,
     // item and let the hardware dispatcher balance them: measured 1.06-2.5x
     // faster than the cap for causal prefill with more tiles than programs.
     const int64_t cap = (int64_t)dev->num_cus * wg_kernel;
-    grid = work < cap ? work : cap;
+    grid = items < cap ? items : cap;
   } else if (req->persistent_programs > 0) {
-    grid = work < req->persistent_programs ? work : req->persistent_programs;
+    grid = items < req->persistent_programs ? items : req->persistent_programs;
   }
   out->grid = (int32_t)grid;
+  out->threads = threads_of(kernel, layout);
   out->arrival_counters = (int32_t)fused_merge_counters(s, layout, splits, rows, tasks);
   return FGW_MHA_OK;
 }

@@ -98,9 +98,10 @@ typedef struct {
                                   single-stage kernel with 4x (or 2x) the splits;
                                   1 or 2 selects the key layout's single-stage (two
                                   workgroups per CU) or double-stage kernel where both exist
-                                  (head-dim tile 128); elsewhere only the kernel's own count
-                                  is accepted. No reference counterpart (a kernel-variant
-                                  choice). */
+                                  (head-dim tile 128; at Sq = 1, where most shapes run the
+                                  single-token variant, it then selects the grid's cap alone);
+                                  elsewhere only the kernel's own count is accepted. No
+                                  reference counterpart (a kernel-variant choice). */
 } fgw_mha_request;
 
 /* Largest batch of a length-balanced split plan (split_keys > 0). */
@@ -115,7 +116,12 @@ typedef struct {
 } fgw_mha_device_info;
 
 /* Resolved launch plan: the attributes the reference launch callable
- * exposes (v7.py:475-487, :500-512) plus workspace sizes. */
+ * exposes (v7.py:475-487, :500-512) plus workspace sizes. rows_per_tile,
+ * q_tiles, query_tile_tasks and work_items are the layout's tiling; grid and
+ * threads are what is launched. A layout has kernel variants, chosen from shape
+ * and plan, of which one differs from that tiling: direct prefill-layout plans
+ * that would leave the chip idle run as items of 128 rows, two to a tile of
+ * 256, on up to twice work_items programs. */
 typedef struct {
   int32_t layout;          /* fgw_mha_layout actually used */
   int32_t rows_per_tile;   /* query rows per work item (reference block_q) */
@@ -123,7 +129,7 @@ typedef struct {
   int32_t num_splits;      /* KV splits per (b, h, q tile) */
   int32_t query_tile_tasks;/* B * H * q_tiles */
   int32_t work_items;      /* query_tile_tasks * num_splits (compute_work) */
-  int32_t grid;            /* launched programs (compute_grid) */
+  int32_t grid;            /* launched programs (compute_grid); each runs its share of the items */
   int32_t threads;         /* threads per program */
   int32_t execution_mode;  /* 0 = direct single split, 1 = split and merge */
   int32_t dim_padded;      /* head-dim tile of the selected kernel */
@@ -132,8 +138,10 @@ typedef struct {
   int32_t split_keys;      /* request.split_keys of a split plan (0: even splits); work_items and
                               the workspaces are then upper bounds, slot s of request b is used
                               for s < clamp(ceil(len_b / split_keys), 1, num_splits) */
-  int32_t stages;          /* K/V stages per key group of the selected kernel (query and key
-                              layouts; the prefill layout's rings have 4 slots: 4) */
+  int32_t stages;          /* K/V stages per key group of the layout's kernel (query and key
+                              layouts; the prefill layout's rings have 4 slots: 4). The
+                              single-token variant (key layout, Sq = 1) has none: there it only
+                              records the choice that num_splits and grid come from */
   int32_t arrival_counters; /* > 0: fgw_mha_fwd can fuse this split plan's merge into the
                               partial kernel when the call supplies an arrival buffer of this
                               many int32 (fgw_mha_tensors.arrivals; one 128-byte counter line

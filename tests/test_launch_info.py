@@ -34,8 +34,10 @@ def launch(b=2, sq=1, h=8, d=128, kv=2048, page=64, causal=0, layout=-1, splits=
 def test_variant_of_a_plan(name, kwargs):
     plan, info = launch(**kwargs)
     assert info.name == name
+    assert (info.grid, info.threads) == (plan.grid, plan.threads)
+    assert info.threads == (512 if name[:4] in ("deco", "pref", "half") or "eight" in name else 256)
     if not name.startswith("half"):
-        assert (info.q_tiles, info.work_items, info.grid) == (plan.q_tiles, plan.work_items, plan.grid)
+        assert (info.q_tiles, info.work_items) == (plan.q_tiles, plan.work_items)
 
 
 MIB = 1 << 20
@@ -97,6 +99,33 @@ def test_device_cap_is_the_selected_kernels_residency():
     assert launch(b=64, h=32, kv=64, stages=2)[0].grid == 256  # asked for
     assert launch(b=64, h=32, kv=64, programs=0)[0].grid == 2048
     assert launch(b=64, h=32, kv=64, programs=300)[0].grid == 300
+
+
+def test_half_tile_grids_keep_the_requested_cap():
+    """The kernel's items are half the plan's tiles; the grid is counted in them."""
+    half = dict(b=1, h=16, sq=1536, kv=1024)  # 96 tiles of 256 rows, 192 items
+    for programs, grid in ((-1, 192), (0, 192), (300, 192), (192, 192), (100, 100), (96, 96), (7, 7)):
+        plan, info = launch(**half, programs=programs)
+        assert (info.name, info.rows_per_item, info.work_items) == ("half_tiles", 128, 192)
+        assert plan.work_items == 96 and plan.grid == info.grid == grid
+    # More items than the CUs: the device cap, but for causal plans.
+    for items, grid, many in ((387, 256, dict(b=3, h=43, sq=257, kv=2048, d=64)),
+                              (312, 312, dict(b=2, h=13, sq=1500, kv=1536, d=64, causal=1))):
+        plan, info = launch(**many)
+        assert (info.name, info.work_items, plan.grid) == ("half_tiles", items, grid)
+
+
+@pytest.mark.parametrize("kwargs", [dict(b=1, h=16, sq=1536, kv=1024), dict(sq=4096), dict(), dict(sq=64)])
+def test_a_grid_beyond_the_items_is_refused(kwargs):
+    plan, info = launch(**kwargs, programs=0)
+    assert plan.grid == info.work_items
+    plan.grid += 1
+    w = -(-kwargs.get("kv", 2048) // 64)
+    b = kwargs.get("b", 2)
+    shape = _lib.Shape(b, kwargs.get("sq", 1), kwargs.get("h", 8), 128, b * w * 64, w, 64, 0,
+                       _lib.DTYPE_BFLOAT16)
+    with pytest.raises(ValueError, match="does not match"):
+        _lib.launch_info(shape, plan)
 
 
 def test_a_plan_of_another_shape_is_refused():
