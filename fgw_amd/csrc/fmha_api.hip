@@ -555,21 +555,23 @@ constexpr int kRowsHalfTile = HCfg<true, 128, kRowsGroup>::ROWS_TILE;
 // rows whose items take `per_step` blocks at a time, at full table capacity:
 // the longest item or an even share of all of them (longest first), plus an
 // item's fixed cost (about five blocks) for each round.
+// Evaluated on every launch: closed sums, no loop over the tiles.
 double critical_steps(const fgw_mha_shape* s, int rows, int per_step, double step_cost) {
   const int64_t capacity = (int64_t)s->width * s->page_size;
   const int q_tiles = (s->sq + rows - 1) / rows;
   const int64_t tiles = (int64_t)s->batch * s->heads * q_tiles;
   const int64_t rounds = (tiles + kNumCus - 1) / kNumCus;
-  auto steps = [&](int64_t vis) {
-    vis = vis < 0 ? 0 : (vis > capacity ? capacity : vis);
-    return (vis + 64 * per_step - 1) / (64 * per_step);
-  };
-  const int64_t longest = steps(capacity);
+  const int64_t step = 64 * per_step;  // keys; rows is a multiple of it
+  const int64_t longest = (capacity + step - 1) / step;
   double path = (double)(rounds * longest);
   if (s->causal) {
-    int64_t sum = 0;
-    for (int t = 0; t < q_tiles; ++t)
-      sum += steps(capacity - s->sq + ((int64_t)(t + 1) * rows < s->sq ? (t + 1) * rows : s->sq));
+    // Tile t of the `full` whole ones sees first + (t + 1) rows keys, none of them
+    // below tile `none`; a partial last tile sees all.
+    const int64_t first = capacity - s->sq, full = s->sq / rows;
+    const int64_t skip = first < 0 ? -first / rows : 0, none = skip < full ? skip : full;
+    const int64_t lead = first < 0 ? -(-first / step) : (first + step - 1) / step;
+    const int64_t sum = (full - none) * lead + rows / step * (full * (full + 1) - none * (none + 1)) / 2 +
+                        (full * rows < s->sq ? longest : 0);
     const double share = (double)sum * s->batch * s->heads / kNumCus;
     path = share > (double)longest ? share : (double)longest;
   }

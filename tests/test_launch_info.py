@@ -1,4 +1,6 @@
 """Which kernel variant a planned call launches (CPU: the choice is host arithmetic)."""
+import random
+
 import pytest
 
 from fgw_amd import _lib
@@ -133,3 +135,36 @@ def test_a_plan_of_another_shape_is_refused():
     other = _lib.Shape(3, 1, 8, 128, 4096, 32, 64, 0, _lib.DTYPE_BFLOAT16)
     with pytest.raises(ValueError, match="does not match"):
         _lib.launch_info(other, plan)
+
+
+def _half_tiles_by_loop(b, sq, h, capacity, causal, dpad):
+    """The rule's definition (half_tiles in fmha_api.hip), tile by tile."""
+    def critical(rows, per_step, cost):
+        q_tiles = -(-sq // rows)
+        rounds = -(-(b * h * q_tiles) // 256)
+        steps = lambda vis: -(-min(max(vis, 0), capacity) // (64 * per_step))  # noqa: E731
+        path = rounds * steps(capacity)
+        if causal:
+            total = sum(steps(capacity - sq + min((t + 1) * rows, sq)) for t in range(q_tiles))
+            path = max(total * b * h / 256, steps(capacity))
+        return path * cost + 5.0 * rounds
+    if b * h * -(-sq // 256) > 512:
+        return False
+    return critical(128, 2, 1.3 if dpad == 64 else 1.66) < 0.95 * critical(256, 1, 1.0)
+
+
+@pytest.mark.parametrize("causal", [0, 1])
+def test_half_tile_rule_over_seeded_shapes(causal):
+    r = random.Random(31 + causal)
+    taken = 0
+    for _ in range(3000):
+        b, h = r.choice((1, 2, 3, 8)), r.choice((1, 2, 5, 8, 16, 32))
+        sq = r.choice((r.randint(1, 600), r.randint(1, 9000), 256 * r.randint(1, 20)))
+        d, page = r.choice((48, 64, 96, 128)), r.choice((16, 64, 128, 272))
+        kv = r.choice((r.randint(1, 3000), r.randint(1, 20000), sq))  # often below Sq
+        _, info = launch(b=b, sq=sq, h=h, d=d, kv=kv, page=page, causal=causal, splits=1,
+                         layout=_lib.LAYOUT_PREFILL)
+        want = _half_tiles_by_loop(b, sq, h, -(-kv // page) * page, causal, 64 if d <= 64 else 128)
+        assert info.name.startswith("half") == want, (b, sq, h, d, kv, page)
+        taken += want
+    assert 300 < taken < 2700
