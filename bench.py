@@ -785,13 +785,17 @@ def main():
         pcall = lambda: dkern.partial_kernel(*dinputs)  # noqa: E731
         p_ms = region_ms(pcall, args.steps, args.warmup) / args.steps
         p_achieved = dbytes / (p_ms * 1e-3) / 1e9
+        variant = dkern.launch_info.name
         stage_name = "single-stage" if dkern.stages == 1 else "double-stage"
+        kernel_name = ("decode_kernel (partial, " if variant == "decode" else
+                       f"fwd_kernel (partial, {variant} variant, {stage_name}, ")
         decode["roofline"] = {"bound": "hbm",
-                              "kernel": f"fwd_kernel (partial, key layout, {stage_name}, "
-                                        f"{dkern.num_splits} splits)",
+                              "kernel": f"{kernel_name}{dkern.num_splits} splits)",
                               "achieved": p_achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                               "frac": p_achieved / PEAK_HBM_GBS,
-                              "traffic": traffic_from_profile("decode_partial"),
+                              # Measured on the key kernel: of no other variant.
+                              "traffic": traffic_from_profile("decode_partial")
+                              if variant == "key" else None,
                               "traffic_source": str(TRAFFIC_SUMMARY.relative_to(ROOT)),
                               "kernel_us": p_ms * 1e3,
                               "kernel_us_source": "back-to-back region of partial-only calls / calls"}
