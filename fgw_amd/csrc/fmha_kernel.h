@@ -187,10 +187,10 @@ struct CMin {
 // (GroupRows); non-temporal loads where stream_kv says so.
 // kStream (key layout): the plain kernel with non-temporal loads where stream_kv
 // says so, for table capacities that can exceed the last-level cache.
-// kDual (query layout, head-dim tile 256): two sets of four waves hold the same
-// 128 query rows, each takes 32 keys of every 64-key block, and their states
-// meet in LDS at the end of an item. At this tile the K/V stages fill a CU's LDS
-// with one workgroup; with four waves every SIMD had one, whose chain of LDS
+// kDual (query layout, D 256, page_size % 64 == 0, so that both halves of a block
+// lie in its page): two sets of four waves hold the same 128 query rows, each
+// takes 32 keys of every 64-key block, and their states meet in LDS at the end of
+// an item. At this tile the K/V stages fill a CU's LDS with one workgroup; with four waves every SIMD had one, whose chain of LDS
 // reads, MFMAs and softmax nothing overlapped (2.6 us per block for 0.9 us of
 // MFMAs). With eight, one set's softmax runs beside the other's MFMAs, at the
 // same LDS and the same loads; what bounds it is still the chain (two waves per
@@ -1337,8 +1337,8 @@ __global__ __launch_bounds__(C::THREADS) void fwd_kernel(FwdParams p_arg,
     auto ids_of = [&](int pos) -> int32_t {
       if constexpr (C::GROUPS)
         return group_id<C>(p, table_b, pos, wq, lane);
-      else  // (DUAL: the second half of the last block may lie past the table)
-        return page_id(p, table_b, C::DUAL && pos >= capacity ? 0 : pos);
+      else
+        return page_id(p, table_b, pos);
     };
     if (p.mode != 2 && !p.causal && !balanced) {
       const int nfull = (capacity + C::BLOCK - 1) / C::BLOCK;
