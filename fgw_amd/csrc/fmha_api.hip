@@ -613,18 +613,19 @@ bool half_tiles(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
 // - Key and query layouts: the row-group kernel where the whole-block fast path
 //   would not hold (pages that a block, 32 keys in the key layout and 64 in the
 //   query layout, straddles, or a head dim below its tile) and an instruction's
-//   rows (512 / tile of them) lie in one page. Measured against the plain kernel:
+//   rows (512 / tile of them) lie in one page; tile 32 also at whole blocks from
+//   128 MiB on (0.94-1.01 of the plain kernel). Measured against the plain kernel:
 //   B4 H16 Q8 KV <= 8192 causal pages of 16 66.7 -> 42.2 us; B8 H32 Q4 KV <= 2048
 //   pages of 16 65.9 -> 39.0; B16 H8 Q20 D96 pages of 48 21.4 -> 15.7; B8 H32 Q5
-//   D32 pages of 16 71.5 -> 38.6. With whole blocks it is the slower one (B64 H8
-//   Sq 8 KV 4096, shared pages, cached loads: 82 us against 72).
+//   D32 pages of 16 71.5 -> 38.6. At whole blocks of the other tiles it is the slower
+//   one (B64 H8 Sq 8 KV 4096 D128, shared pages, cached loads: 82 us against 72).
 // - Query layout: the eight-wave kernel where dual_takes it.
 // - Prefill layout: a row-group variant where the whole-block fast path would
 //   not hold (pages that a 64-key block straddles, or a head dim below its
 //   tile) and an instruction's rows (512 / tile of them) still lie in one page;
 //   the half-tile kernel where half_tiles takes the plan.
-constexpr int64_t kCacheBytes = int64_t(256) << 20;      // last-level cache
-constexpr int64_t kDecodeMaxBytes = int64_t(128) << 20;  // decode_kernel at tile 128, whole blocks
+constexpr int64_t kCacheBytes = int64_t(256) << 20;  // last-level cache
+constexpr int64_t kLargeBytes = int64_t(128) << 20;  // whole blocks: other kernels from here on
 
 // K and V bytes that the call's items read at full table capacity, and of the
 // rows they lie in (requests may share pages: not more than the pool's).
@@ -649,10 +650,11 @@ Kernel kernel_of(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
   const int64_t bytes = capacity_bytes(s);
   if (key && s->sq == 1 &&
       decode_takes(p->dim_padded, (int64_t)s->heads * s->dim * 2, s->page_size) &&
-      !(whole && ((p->dim_padded == 128 && bytes >= kDecodeMaxBytes) ||
+      !(whole && ((p->dim_padded == 128 && bytes >= kLargeBytes) ||
                   (p->dim_padded == 64 && bytes >= kCacheBytes))))
     return kKernelDecode;
-  if (row_groups && !whole) return key ? kKernelKeyGroups : kKernelQueryGroups;
+  if (row_groups && (!whole || (key && p->dim_padded == 32 && bytes >= kLargeBytes)))
+    return key ? kKernelKeyGroups : kKernelQueryGroups;
   if (key && p->q_tiles == 1 && p->dim_padded >= 64 && max_kv_bytes(s) > kCacheBytes)
     return kKernelKeyStream;
   if (dual_takes(s, p)) return kKernelQueryDual;
@@ -968,12 +970,19 @@ int fgw_mha_plan(const fgw_mha_shape* s, const fgw_mha_request* req,
 
   const int64_t items = items_of(s, out, kernel);
   int64_t grid = items;
-  if (req->persistent_programs == -1 && !s->causal) {
+  if (req->persistent_programs == -1 && !s->causal && !(decode && split_keys == 0)) {
     // Device cap: the resident workgroups of all CUs loop over contiguous
     // ranges of work items. Causal work items differ in size (and with
     // Sq > len many are empty), so causal plans keep one workgroup per work
     // item and let the hardware dispatcher balance them: measured 1.06-2.5x
     // faster than the cap for causal prefill with more tiles than programs.
+    // So do the single-token kernel's, which share nothing from one item to the
+    // next: at the key kernel's one per CU many short items ran one after the
+    // other, and two fixed programs per CU share some counts out unevenly (256 / 512
+    // programs / one per item: B56 H32 KV 512 D32 33.9 / 33.6 / 24.5 us, B56 H32 KV 512
+    // D64 54.5 / 60.0 / 47.0, B48 H32 KV 96 D128 pages of 16 22.3 / 16.8 / 18.7;
+    // geometric mean of 208 shapes 0.786 / 0.740 / 0.714 of the key kernel). Their
+    // length-balanced plans count items that may not exist, and keep the cap.
     const int64_t cap = (int64_t)dev->num_cus * wg_kernel;
     grid = items < cap ? items : cap;
   } else if (req->persistent_programs > 0) {

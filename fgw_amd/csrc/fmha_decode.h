@@ -422,12 +422,7 @@ __global__ __launch_bounds__(C::THREADS, 4) void decode_kernel(FwdParams p_arg,
   }
 }
 
-// Resident workgroups per CU (the launch bound's registers; LDS allows more), and
-// the programs per CU of a capped grid. With one per CU, as the key kernel has at
-// tile 128, many short items ran one after the other: B64 H32 KV 512 D 32 51.8 us
-// (the key kernel 48.7), with two 39.9; KV 128 D 64 25.7 -> 17.9; B64 H8 KV 4096 pages
-// of 16, shared, 81.3 -> 64.7. Long items do not need it (0.97-1.02; D 64 pages of
-// 16, B32 H16 KV 8192 shared 87.8 -> 97.8).
+// Resident workgroups per CU (the launch bound's registers; LDS allows more).
 constexpr int kDecodeWgPerCu = 2;
 
 // Shapes this kernel takes: load instructions whose rows lie in one page and

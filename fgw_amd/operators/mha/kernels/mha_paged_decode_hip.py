@@ -249,7 +249,8 @@ def build_kernel(batch, sq, heads, dim, pool_rows, width, page_size, causal, dty
 
     Arguments follow the reference build_kernel (v7.py:32-47) plus
     persistent_programs (v7_experimental.py:29-30: None = uncapped grid; here
-    the default caps the grid at the device's resident workgroups),
+    the default caps the grid at the device's resident workgroups, but for
+    causal plans and single-token items, which the hardware balances better),
     cache_lengths (host-known lengths for the cost model,
     cube_general.py:17, :45) and layout ("query" = 4 waves split 128 query
     rows; "prefill" = 8 waves split 256 query rows in two groups that

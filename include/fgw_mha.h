@@ -77,7 +77,8 @@ typedef struct {
  * (v7.py:43-46, :94-113; v7_experimental.py:29-30 persistent_programs). */
 typedef struct {
   int32_t num_splits;          /* 0 = automatic; else 1,2,4,...,128 */
-  int32_t persistent_programs; /* -1 = CU-derived cap (uncapped for causal), 0 = uncapped grid, n > 0 = cap */
+  int32_t persistent_programs; /* -1 = CU-derived cap (none for causal plans and for the
+                                  single-token kernel's even splits), 0 = uncapped grid, n > 0 = cap */
   int32_t layout;              /* fgw_mha_layout */
   int32_t split_keys;          /* 0 = every request's keys split evenly into num_splits; > 0 =
                                   splits balanced by length (key layout, num_splits > 1, B <=
@@ -190,7 +191,8 @@ int fgw_mha_query_device(int device, fgw_mha_device_info* info);
  * prefill layout, four in the query layout from 2^22 query-key pairs).
  * Stages: the layout's default kernel unless requested or the automatic
  * short-decode rule selects the key layout's single-stage kernel; the
- * persistent grid is capped at the selected kernel's resident slots. Errors
+ * CU-derived cap is the selected kernel's resident slots (of the named stage
+ * count's key kernel where the request names one). Errors
  * mirror the reference ValueErrors (v7.py:49-55, :97-99). */
 int fgw_mha_plan(const fgw_mha_shape* shape, const fgw_mha_request* request,
                  const fgw_mha_device_info* device, fgw_mha_plan_t* plan);

@@ -58,6 +58,9 @@ MIB = 1 << 20
     ("decode", 0, dict(page=16, kv=16384)), ("decode", 128, dict(page=16, kv=16400)),
     ("decode", 128, dict(d=192, kv=65536)), ("decode", 128, dict(d=256, kv=65536)),
     ("key_groups", 128, dict(sq=8, page=16, kv=16400)),
+    # Tile 32: row groups for whole blocks from 128 MiB on, cached loads.
+    ("key", 0, dict(sq=8, d=32, kv=65472)), ("key_groups", 0, dict(sq=8, d=32, kv=65536)),
+    ("decode", 0, dict(d=32, kv=131072)),
     # Heads that share 128-byte lines, and more than one query tile: never.
     ("decode", 0, dict(d=80, kv=65536)), ("key_groups", 0, dict(sq=8, d=96, kv=65536)),
     ("query_groups", 128, dict(sq=128, page=16, kv=32768, layout=0)),
@@ -94,9 +97,11 @@ def test_order_of_causal_items(first, kwargs):
 
 
 def test_device_cap_is_the_selected_kernels_residency():
-    """Two single-token programs per CU; one of the double-stage key kernel's."""
-    assert launch(b=64, h=32, kv=64)[0].grid == 512
-    assert launch(b=64, h=32, kv=256, d=64)[0].grid == 512
+    """One program per item of the single-token kernel, two per CU for length-balanced splits
+    (whose items may not exist); one per CU of the double-stage key kernel."""
+    assert launch(b=64, h=32, kv=64)[0].grid == 2048
+    assert launch(b=64, h=32, kv=256, d=64)[0].grid == 2048
+    assert launch(b=64, h=8, kv=256, splits=8, split_keys=64)[0].grid == 512
     assert launch(b=64, h=32, kv=64, page=6)[0].grid == 256  # the key kernel
     assert launch(b=64, h=32, kv=64, stages=2)[0].grid == 256  # asked for
     assert launch(b=64, h=32, kv=64, programs=0)[0].grid == 2048
