@@ -607,7 +607,12 @@ bool half_tiles(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
 //   1.14 from 256 MiB; 0.88-1.01 below. At 64 it is the last-level cache's size
 //   (the key kernel gains more from non-temporal loads): 0.97-1.02 and 0.65-0.99
 //   with shared pages below, 1.00-1.24 from there on. Tiles 32 (0.6-0.97) and 256
-//   (0.72-1.06) have no such line.
+//   (0.72-1.06) have no such line. Nor for a few long items (explicit small split
+//   counts), whose time is one workgroup's own stream: at tile 128 from 2048 keys an
+//   item (1.01-1.06 there, 1.10 at 4096, 1.17 at 16384; 0.95-1.02 at 1024), at 256
+//   from 1024 keys with up to 8 items (1.07), 128 more for each further one (16 items
+//   of 2048 keys 1.04, 64 of 4096 0.99, 128 of 2048 0.90); tiles 32 and 64 gain there
+//   (0.57-0.76).
 // - Key layout: the kernel with non-temporal loads where the table can hold more K/V
 //   than the last-level cache.
 // - Key and query layouts: the row-group kernel where the whole-block fast path
@@ -637,6 +642,16 @@ int64_t max_kv_bytes(const fgw_mha_shape* s) {
   return pool < capacity_bytes(s) ? pool : capacity_bytes(s);
 }
 
+bool large_for_decode(int dpad, int64_t bytes) {
+  return (dpad == 128 && bytes >= kLargeBytes) || (dpad == 64 && bytes >= kCacheBytes);
+}
+bool long_for_decode(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
+  const int64_t capacity = (int64_t)s->width * s->page_size;
+  const int64_t keys = p->split_keys > 0 ? p->split_keys : capacity / p->num_splits;
+  return (p->dim_padded == 128 && keys >= 2048) ||
+         (p->dim_padded == 256 && keys >= 128 * (int64_t)(p->work_items > 8 ? p->work_items : 8));
+}
+
 Kernel kernel_of(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
   const bool row_groups = s->page_size % (512 / p->dim_padded) == 0;
   const bool padded = s->dim != p->dim_padded;
@@ -650,8 +665,7 @@ Kernel kernel_of(const fgw_mha_shape* s, const fgw_mha_plan_t* p) {
   const int64_t bytes = capacity_bytes(s);
   if (key && s->sq == 1 &&
       decode_takes(p->dim_padded, (int64_t)s->heads * s->dim * 2, s->page_size) &&
-      !(whole && ((p->dim_padded == 128 && bytes >= kLargeBytes) ||
-                  (p->dim_padded == 64 && bytes >= kCacheBytes))))
+      !(whole && (large_for_decode(p->dim_padded, bytes) || long_for_decode(s, p))))
     return kKernelDecode;
   if (row_groups && (!whole || (key && p->dim_padded == 32 && bytes >= kLargeBytes)))
     return key ? kKernelKeyGroups : kKernelQueryGroups;

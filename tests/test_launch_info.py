@@ -53,6 +53,11 @@ MIB = 1 << 20
     # Tile 64: the single-token kernel below the cache's size.
     ("decode", 0, dict(d=64, kv=65472)), ("key", 0, dict(d=64, kv=65536)),
     ("key_stream", 256, dict(d=64, kv=65600)),
+    # A few long items: the key kernel at tiles 128 and 256.
+    ("decode", 0, dict(kv=8192, splits=8)), ("key", 0, dict(kv=8192, splits=4)),
+    ("key", 0, dict(kv=8192, splits=16, split_keys=2048)), ("decode", 0, dict(kv=8192, d=64, splits=1)),
+    ("key", 0, dict(b=1, h=1, kv=1024, d=256, splits=1)), ("decode", 0, dict(kv=2048, d=256, splits=2)),
+    ("decode", 0, dict(kv=8192, page=16, splits=1)),
     # Small pages, padded head dims and D 256: the same kernel at any size, past the
     # cache from half of it.
     ("decode", 0, dict(page=16, kv=16384)), ("decode", 128, dict(page=16, kv=16400)),
