@@ -265,7 +265,11 @@ bool has_key_single(int layout, int dpad) { return layout == kLayoutKey && dpad 
 // B2 H8 Q8 / Q16 at 2x (32 splits): KV 32768 0.976x / 0.975x, KV 8192
 // 0.969x / 0.966x, where 4x (64 splits) lost at Q16 (1.03x); below 16
 // splits (B2 H16 or B8 H8, 4-8 splits) it measured 1.00-1.05x, so those
-// plans stay.
+// plans stay. These are the key kernel's figures; at Sq 1 the single-token kernel
+// runs the same plans where kernel_of takes it, within 1-4% of its best count (three
+// rotating sets, automatic / best of 1-128): B2 H8 KV 8192 17.2 / 17.1 us, B1 H8 KV
+// 16384 17.6 / 17.3, B2 H8 KV 32768 pages of 16 47.2 / 47.1, D 64 B2 H8 KV 16384 pages
+// of 16 18.6 / 17.8.
 int single_stage_splits(const fgw_mha_shape* s, const fgw_mha_device_info* dev, int layout,
                         int dpad, int64_t tasks, int splits, int64_t capacity) {
   if (!has_key_single(layout, dpad) || s->sq > 16 || splits < 16 ||
